@@ -2667,186 +2667,6 @@ gb_tuple_size(cplan *P, const Lane &L)
     return t_hoff + ROWID_SIZE;
 }
 
-__device__ __forceinline__ bool
-gb_keys_match(cplan *P, const Lane &L, const kern_tupitem *t)
-{
-    const char *base = (const char *)t;
-    uint32_t pos = P->gb_t_hoff + P->gb_states_end;
-    for (int j = 0; j < (int)P->gb_nattrs; j++)
-    {
-        xagg ag = P->aggs[j];
-        if (ag.action != KAGG_ACTION__VREF)
-            continue;
-        xattr ka = P->keys[ag.key_index];
-        pos = (uint32_t)xalign(ka.attalign, pos);
-        bool tnull = !((t->t_bits[j >> 3] >> (j & 7)) & 1);
-        bool lnull = RNULL(L, ka.reg);
-        if (tnull || lnull)
-        {
-            if (tnull != lnull)
-                return false;   /* NULLs group together (kmode_compare_nulls) */
-            continue;
-        }
-        const char *p = base + pos;
-        int64_t v = L.R[ka.reg];
-        switch (ka.width)
-        {
-            case 1: if (*(const int8_t *)p != (int8_t)v) return false; pos += 1; break;
-            case 2: if (*(const int16_t *)p != (int16_t)v) return false; pos += 2; break;
-            case 4:
-                if (ka.domain == XD_F32)
-                {
-                    if (!fcmp(XC_EQ, (double)__int_as_float(*(const int32_t *)p), (double)as_f32(v)))
-                        return false;
-                }
-                else if (*(const int32_t *)p != (int32_t)v)
-                    return false;
-                pos += 4;
-                break;
-            case 8:
-                if (ka.domain == XD_F64)
-                {
-                    if (!fcmp(XC_EQ, __longlong_as_double(*(const int64_t *)p), as_f64(v)))
-                        return false;
-                }
-                else if (*(const int64_t *)p != v)
-                    return false;
-                pos += 8;
-                break;
-            default:
-            {
-                if (ka.domain == XD_NUM)
-                {
-                    /* numeric keys group by value (xpu_numeric_datum_comp) */
-                    xnum x, y;
-                    if (num_parse((const uint8_t *)p, &x) || num_read(L, ka.reg, &y) ||
-                        num_compare(x, y) != 0)
-                        return false;
-                    pos += varsize_any((const uint8_t *)p);
-                    break;
-                }
-                uint32_t len = (uint32_t)L.R[ka.reg + 1];
-                uint32_t hdr = *(const uint32_t *)p;
-                if (((hdr >> 2) & 0x3fffffff) != len + 4)
-                    return false;
-                const uint8_t *s = (const uint8_t *)(uintptr_t)v;
-                for (uint32_t i = 0; i < len; i++)
-                    if ((uint8_t)p[4 + i] != s[i])
-                        return false;
-                pos += 4 + len;
-                break;
-            }
-        }
-    }
-    return true;
-}
-
-__device__ __forceinline__ void
-gb_tuple_write(cplan *P, const Lane &L, kern_hashitem *hi, uint32_t unit,
-               uint32_t hash, uint32_t rowid, uint64_t next)
-{
-    char *ubuf = (char *)hi;
-    for (uint32_t i = 0; i < unit; i += 8)
-        *(uint64_t *)(ubuf + i) = 0;
-    hi->next = next;
-    char *buf = (char *)&hi->t;
-    kern_tupitem *t = &hi->t;
-    uint16_t infomask = HEAP_HASNULL;
-    uint8_t *bits = t->t_bits;
-    uint32_t nattrs = P->gb_nattrs;
-    uint32_t t_hoff = P->gb_t_hoff;
-    /* partial states, in their initial values */
-    for (int j = 0; j < (int)nattrs; j++)
-    {
-        xagg ag = P->aggs[j];
-        if (ag.action == KAGG_ACTION__VREF)
-            continue;
-        char *s = buf + t_hoff + ag.state_off;
-        bits[j >> 3] |= (uint8_t)(1 << (j & 7));
-        switch (ag.action)
-        {
-            case KAGG_ACTION__NROWS_ANY:
-            case KAGG_ACTION__NROWS_COND:
-                break;
-            case KAGG_ACTION__PMIN_INT32: case KAGG_ACTION__PMIN_INT64:
-                *(int32_t *)s = ag.state_size << 2;
-                *(int64_t *)(s + 8) = INT64_MAX;
-                infomask |= HEAP_HASVARWIDTH;
-                break;
-            case KAGG_ACTION__PMAX_INT32: case KAGG_ACTION__PMAX_INT64:
-                *(int32_t *)s = ag.state_size << 2;
-                *(int64_t *)(s + 8) = INT64_MIN;
-                infomask |= HEAP_HASVARWIDTH;
-                break;
-            case KAGG_ACTION__PMIN_FP64:
-                *(int32_t *)s = ag.state_size << 2;
-                *(double *)(s + 8) = 1.7976931348623157e308;
-                infomask |= HEAP_HASVARWIDTH;
-                break;
-            case KAGG_ACTION__PMAX_FP64:
-                *(int32_t *)s = ag.state_size << 2;
-                *(double *)(s + 8) = -1.7976931348623157e308;
-                infomask |= HEAP_HASVARWIDTH;
-                break;
-            case KAGG_ACTION__PSUM_NUMERIC: case KAGG_ACTION__PAVG_NUMERIC:
-                /* attrs: the sum's scale (cuda_gpupreagg.cu:173-183) */
-                *(int32_t *)s = ag.state_size << 2;
-                *(uint32_t *)(s + 4) = ag.num_scale;
-                infomask |= HEAP_HASVARWIDTH;
-                break;
-            default:
-                *(int32_t *)s = ag.state_size << 2;
-                infomask |= HEAP_HASVARWIDTH;
-                break;
-        }
-    }
-    /* grouping keys */
-    uint32_t pos = t_hoff + P->gb_states_end;
-    for (int j = 0; j < (int)nattrs; j++)
-    {
-        xagg ag = P->aggs[j];
-        if (ag.action != KAGG_ACTION__VREF)
-            continue;
-        xattr ka = P->keys[ag.key_index];
-        pos = (uint32_t)xalign(ka.attalign, pos);
-        if (RNULL(L, ka.reg))
-            continue;
-        bits[j >> 3] |= (uint8_t)(1 << (j & 7));
-        char *p = buf + pos;
-        int64_t v = L.R[ka.reg];
-        switch (ka.width)
-        {
-            case 1: *(int8_t *)p = (int8_t)v; pos += 1; break;
-            case 2: *(int16_t *)p = (int16_t)v; pos += 2; break;
-            case 4: *(int32_t *)p = (int32_t)v; pos += 4; break;
-            case 8: *(int64_t *)p = v; pos += 8; break;
-            default:
-            {
-                if (ka.domain == XD_NUM)
-                {
-                    pos += num_reg_varlena_write(L, ka.reg, (uint8_t *)p);
-                    infomask |= HEAP_HASVARWIDTH;
-                    break;
-                }
-                uint32_t len = (uint32_t)L.R[ka.reg + 1];
-                const uint8_t *s = (const uint8_t *)(uintptr_t)v;
-                *(uint32_t *)p = (len + 4) << 2;
-                for (uint32_t i = 0; i < len; i++)
-                    p[4 + i] = s[i];
-                pos += 4 + len;
-                break;
-            }
-        }
-    }
-    pos += ROWID_SIZE;
-    t->t_len = pos;
-    t->hash = hash;
-    t->t_infomask2 = (uint16_t)(nattrs & HEAP_NATTS_MASK);
-    t->t_infomask = infomask;
-    t->t_hoff = (uint8_t)(t_hoff + MINIMAL_TUPLE_OFFSET);
-    *(uint32_t *)(buf + pos - ROWID_SIZE) = rowid;
-}
-
 /* LDS partial table: struct of arrays over n entries (layout in xplan) */
 struct LdsTable
 {
@@ -2867,6 +2687,429 @@ lds_table_at(cplan *P, unsigned long long *base, uint32_t n)
     T.rows = (uint32_t *)(T.f64 + (uint64_t)P->lds_n64 * n);
     T.f32 = T.rows + n;
     return T;
+}
+
+/* Device-coherent accesses to group tuples.  A group tuple is written by one
+ * lane and read by lanes of other XCDs while the kernel runs; every store of
+ * the tuple and every load of it on the lookup path goes past the XCD's own
+ * L2 (relaxed, agent scope), so publishing needs only the stores' completion
+ * and a lookup needs no fence.  A release / acquire pair per group writes back
+ * and invalidates a whole L2 each time: the dump merge that inserts the
+ * 10,000 groups of a 100M-row group-by took 1.47 ms with it, 0.98 ms without,
+ * and 0.19 ms with shared reservations and gathered entries (gb_alloc,
+ * lds_flush). */
+template <typename T>
+__device__ __forceinline__ void
+gst(void *p, T v)
+{
+    __hip_atomic_store((T *)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <typename T>
+__device__ __forceinline__ T
+gld(const void *p)
+{
+    return __hip_atomic_load((const T *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* numeric grouping keys are varlena images written and compared byte by byte
+ * with plain accesses: such plans publish with a release and confirm a miss
+ * after an acquire */
+__device__ __forceinline__ bool
+gb_num_keys(cplan *P)
+{
+    bool num = false;
+    for (int k = 0; k < (int)P->nkeys; k++)
+        num = num || P->keys[k].domain == XD_NUM;
+    return num;
+}
+
+/* whether the group tuple holds the key registers' values.  Written without
+ * early exits: the answer is one flag every lane computes to the end, not a
+ * value carried out of divergent branches. */
+__device__ __forceinline__ bool
+gb_keys_match(cplan *P, const Lane &L, const kern_tupitem *t)
+{
+    const char *base = (const char *)t;
+    uint32_t pos = P->gb_t_hoff + P->gb_states_end;
+    bool same = true;
+    for (int j = 0; j < (int)P->gb_nattrs; j++)
+    {
+        xagg ag = P->aggs[j];
+        if (ag.action != KAGG_ACTION__VREF)
+            continue;
+        xattr ka = P->keys[ag.key_index];
+        pos = (uint32_t)xalign(ka.attalign, pos);
+        const bool tnull = !((gld<uint8_t>(&t->t_bits[j >> 3]) >> (j & 7)) & 1);
+        const bool lnull = RNULL(L, ka.reg);
+        same = same && tnull == lnull;      /* NULLs group together (kmode_compare_nulls) */
+        if (tnull || lnull)
+            continue;
+        const char *p = base + pos;
+        const int64_t v = L.R[ka.reg];
+        switch (ka.width)
+        {
+            case 1: same = same && gld<int8_t>(p) == (int8_t)v; pos += 1; break;
+            case 2: same = same && gld<int16_t>(p) == (int16_t)v; pos += 2; break;
+            case 4:
+                if (ka.domain == XD_F32)
+                    same = same && fcmp(XC_EQ, (double)__int_as_float(gld<int32_t>(p)),
+                                        (double)as_f32(v));
+                else
+                    same = same && gld<int32_t>(p) == (int32_t)v;
+                pos += 4;
+                break;
+            case 8:
+                if (ka.domain == XD_F64)
+                    same = same && fcmp(XC_EQ, __longlong_as_double(gld<int64_t>(p)), as_f64(v));
+                else
+                    same = same && gld<int64_t>(p) == v;
+                pos += 8;
+                break;
+            default:
+            {
+                if (ka.domain == XD_NUM)
+                {
+                    /* numeric keys group by value (xpu_numeric_datum_comp) */
+                    xnum x, y;
+                    same = same && !num_parse((const uint8_t *)p, &x) &&
+                           !num_read(L, ka.reg, &y) && num_compare(x, y) == 0;
+                    pos += varsize_any((const uint8_t *)p);
+                    break;
+                }
+                const uint32_t len = (uint32_t)L.R[ka.reg + 1];
+                const uint8_t *s = (const uint8_t *)(uintptr_t)v;
+                uint32_t hdr;
+                if (ka.attalign >= 4)
+                    hdr = gld<uint32_t>(p);
+                else
+                {
+                    hdr = 0;
+                    for (uint32_t i = 0; i < 4; i++)
+                        hdr |= (uint32_t)gld<uint8_t>(p + i) << (8 * i);
+                }
+                const uint32_t tlen = ((hdr >> 2) & 0x3fffffff) - 4;
+                same = same && tlen == len;
+                const uint32_t n = same ? len : 0;
+                uint32_t diff = 0;
+                if (ka.attalign >= 4)
+                {
+                    /* four characters of the group at a time */
+                    for (uint32_t i = 0; i < n; i += 4)
+                    {
+                        const uint32_t k = n - i < 4 ? n - i : 4;
+                        uint32_t x = 0;
+                        for (uint32_t c = 0; c < k; c++)
+                            x |= (uint32_t)s[i + c] << (8 * c);
+                        diff |= (gld<uint32_t>(p + 4 + i) ^ x) & (~0U >> (32 - 8 * k));
+                    }
+                }
+                else
+                {
+                    for (uint32_t i = 0; i < n; i++)
+                        diff |= (uint32_t)(gld<uint8_t>(p + 4 + i) ^ s[i]);
+                }
+                same = same && diff == 0;
+                pos += 4 + tlen;
+                break;
+            }
+        }
+    }
+    return same;
+}
+
+/* the payload of a group tuple after its states, gathered into 8-byte words
+ * (each stored once, device-coherent); pos: bytes from the tuple's start */
+struct GbWords
+{
+    char       *base;
+    uint32_t    pos;
+    uint64_t    w;
+
+    /* n <= 8 bytes of v (whose other bits are zero) */
+    __device__ __forceinline__ void
+    put(uint64_t v, uint32_t n)
+    {
+        const uint32_t sh = 8 * (pos & 7);
+        w |= v << sh;
+        if ((pos & 7) + n >= 8)
+        {
+            gst<uint64_t>(base + (pos & ~7U), w);
+            w = sh ? v >> (64 - sh) : 0;
+        }
+        pos += n;
+    }
+    /* zero bytes up to offset to */
+    __device__ __forceinline__ void
+    pad(uint32_t to)
+    {
+        while (pos < to)
+        {
+            const uint32_t n = 8 - (pos & 7);
+            put(0, n < to - pos ? n : to - pos);
+        }
+    }
+};
+
+/* whether a new group's tuple can be written with its first contribution in
+ * its states (numeric sums merge it afterwards) */
+__device__ __forceinline__ bool
+gb_init_merged(cplan *P)
+{
+    bool ok = true;
+    for (int j = 0; j < (int)P->gb_nattrs; j++)
+        ok = ok && P->aggs[j].action != KAGG_ACTION__PSUM_NUMERIC &&
+             P->aggs[j].action != KAGG_ACTION__PAVG_NUMERIC;
+    return ok;
+}
+
+/* the 8-byte words of aggregate ag's state after its initial value
+ * (cuda_gpupreagg.cu:18-223) has taken one contribution: the row in the
+ * registers, LDS entry lds_slot of T, or state words src of another tuple -
+ * what gb_merge_global / gb_merge_tuple would leave there, without their
+ * atomics (nine per group of a five-aggregate query).  first: false leaves
+ * the initial value. */
+__device__ __forceinline__ void
+gb_first_state(const xagg &ag, const Lane &L, const LdsTable *T, int lds_slot, const uint64_t *src,
+               bool first, uint64_t (&w)[4])
+{
+    const bool from_lds = lds_slot >= 0;
+    w[0] = (uint64_t)((uint32_t)ag.state_size << 2);
+    w[1] = w[2] = w[3] = 0;
+    switch (ag.action)
+    {
+        case KAGG_ACTION__NROWS_ANY: case KAGG_ACTION__NROWS_COND:
+            w[0] = 0; break;
+        case KAGG_ACTION__PMIN_INT32: case KAGG_ACTION__PMIN_INT64:
+            w[1] = (uint64_t)INT64_MAX; break;
+        case KAGG_ACTION__PMAX_INT32: case KAGG_ACTION__PMAX_INT64:
+            w[1] = (uint64_t)INT64_MIN; break;
+        case KAGG_ACTION__PMIN_FP64:
+            w[1] = (uint64_t)__double_as_longlong(1.7976931348623157e308); break;
+        case KAGG_ACTION__PMAX_FP64:
+            w[1] = (uint64_t)__double_as_longlong(-1.7976931348623157e308); break;
+        case KAGG_ACTION__PSUM_NUMERIC: case KAGG_ACTION__PAVG_NUMERIC:
+            /* attrs: the sum's scale (cuda_gpupreagg.cu:173-183) */
+            w[0] |= (uint64_t)ag.num_scale << 32; return;
+    }
+    if (!first)
+        return;
+    uint64_t rows = 0, f64 = 0, f64b = 0;
+    uint32_t f32 = 0;
+    int64_t iv = 0;
+    double fv = 0.0;
+    bool has = from_lds;
+    if (src)
+    {
+        /* the same layout: its count or value, then two more words */
+        if (ag.action == KAGG_ACTION__NROWS_ANY || ag.action == KAGG_ACTION__NROWS_COND)
+            w[0] = src[0];
+        else
+        {
+            w[0] |= src[0] & ~0xffffffffULL;
+            w[1] = src[1];
+            w[2] = ag.state_size > 16 ? src[2] : 0;
+            w[3] = ag.state_size > 24 ? src[3] : 0;
+        }
+        return;
+    }
+    if (from_lds)
+    {
+        rows = T->rows[lds_slot];
+        if (rows == 0)
+            return;
+        if (ag.lds64 >= 0)
+            f64 = T->f64[(uint64_t)ag.lds64 * T->n + lds_slot];
+        if (ag.action == KAGG_ACTION__STDDEV)
+            f64b = T->f64[(uint64_t)(ag.lds64 + 1) * T->n + lds_slot];
+        if (ag.lds32 >= 0)
+            f32 = T->f32[(uint64_t)ag.lds32 * T->n + lds_slot];
+    }
+    else
+    {
+        if (ag.filter_reg != 0xff && (RNULL(L, ag.filter_reg) || L.R[ag.filter_reg] == 0))
+            return;
+        if (ag.arg_reg != 0xff && !RNULL(L, ag.arg_reg))
+        {
+            has = true;
+            iv = val_as_i64(ag.arg_domain, L.R[ag.arg_reg]);
+            fv = val_as_f64(ag.arg_domain, L.R[ag.arg_reg]);
+        }
+        rows = has ? 1 : 0;
+    }
+    switch (ag.action)
+    {
+        case KAGG_ACTION__NROWS_ANY:
+            w[0] = from_lds ? rows : 1;
+            break;
+        case KAGG_ACTION__NROWS_COND:
+            w[0] = rows;
+            break;
+        case KAGG_ACTION__PMIN_INT32: case KAGG_ACTION__PMIN_INT64:
+        case KAGG_ACTION__PMAX_INT32: case KAGG_ACTION__PMAX_INT64:
+            if (has)
+            {
+                w[0] |= (uint64_t)__PAGG_MINMAX_ATTRS__VALID << 32;
+                w[1] = !from_lds ? (uint64_t)iv
+                     : ag.lds32 >= 0 ? (uint64_t)(int64_t)(int32_t)f32 : f64;
+            }
+            break;
+        case KAGG_ACTION__PMIN_FP64: case KAGG_ACTION__PMAX_FP64:
+            if (has)
+            {
+                const double v = from_lds ? __longlong_as_double((long long)f64) : fv;
+                const double was = __longlong_as_double((long long)w[1]);
+                const bool take = ag.action == KAGG_ACTION__PMIN_FP64 ? v < was : v > was;
+                w[0] |= (uint64_t)__PAGG_MINMAX_ATTRS__VALID << 32;
+                if (take)
+                    w[1] = (uint64_t)__double_as_longlong(v);
+            }
+            break;
+        case KAGG_ACTION__PSUM_INT: case KAGG_ACTION__PAVG_INT:
+            w[1] = rows;
+            w[2] = from_lds ? f64 : (uint64_t)iv;
+            break;
+        case KAGG_ACTION__PSUM_INT64: case KAGG_ACTION__PAVG_INT64:
+        {
+            w[1] = rows;
+            if (from_lds)
+            {
+                const uint64_t sub = (uint64_t)f32 << 32;
+                w[2] = f64 - sub;
+                w[3] = f64 < sub ? ~0ULL : 0ULL;
+            }
+            else
+            {
+                w[2] = (uint64_t)iv;
+                w[3] = iv < 0 ? ~0ULL : 0ULL;
+            }
+            break;
+        }
+        case KAGG_ACTION__PSUM_FP: case KAGG_ACTION__PAVG_FP:
+            w[1] = rows;
+            w[2] = (uint64_t)__double_as_longlong(0.0 + (from_lds ? __longlong_as_double((long long)f64) : fv));
+            break;
+        case KAGG_ACTION__STDDEV:
+            w[1] = rows;
+            w[2] = (uint64_t)__double_as_longlong(0.0 + (from_lds ? __longlong_as_double((long long)f64) : fv));
+            w[3] = (uint64_t)__double_as_longlong(0.0 + (from_lds ? __longlong_as_double((long long)f64b) : fv * fv));
+            break;
+    }
+}
+
+/* writes a new group tuple, every byte of its unit once; first: with the
+ * lane's contribution in its states, else with their initial values */
+__device__ __forceinline__ void
+gb_tuple_write(cplan *P, const Lane &L, kern_hashitem *hi, uint32_t unit,
+               uint32_t hash, uint32_t rowid, uint64_t next, const LdsTable *T, int lds_slot,
+               const kern_tupitem *src, bool first)
+{
+    char *buf = (char *)&hi->t;
+    uint16_t infomask = HEAP_HASNULL;
+    uint64_t bits = 0;              /* attribute j is not NULL (XP_MAX_PROJ <= 64) */
+    const uint32_t nattrs = P->gb_nattrs;
+    const uint32_t t_hoff = P->gb_t_hoff;
+    gst<uint64_t>(&hi->next, next);
+    /* partial states */
+    for (int j = 0; j < (int)nattrs; j++)
+    {
+        xagg ag = P->aggs[j];
+        if (ag.action == KAGG_ACTION__VREF)
+            continue;
+        char *s = buf + t_hoff + ag.state_off;
+        bits |= 1ULL << j;
+        if (ag.action != KAGG_ACTION__NROWS_ANY && ag.action != KAGG_ACTION__NROWS_COND)
+            infomask |= HEAP_HASVARWIDTH;
+        uint64_t w[4];
+        gb_first_state(ag, L, T, lds_slot,
+                       src ? (const uint64_t *)((const char *)src + t_hoff + ag.state_off) : nullptr,
+                       first, w);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++)
+            if (8 * k < ag.state_size)
+                gst<uint64_t>(s + 8 * k, w[k]);
+    }
+    /* grouping keys */
+    uint32_t pos = t_hoff + P->gb_states_end;
+    const bool num = gb_num_keys(P);
+    GbWords W = {buf, pos, 0};
+    if (num)
+    {
+        for (uint32_t i = offsetof(kern_hashitem, t) + pos; i < unit; i += 8)
+            *(uint64_t *)((char *)hi + i) = 0;
+    }
+    for (int j = 0; j < (int)nattrs; j++)
+    {
+        xagg ag = P->aggs[j];
+        if (ag.action != KAGG_ACTION__VREF)
+            continue;
+        xattr ka = P->keys[ag.key_index];
+        pos = (uint32_t)xalign(ka.attalign, pos);
+        if (!num)
+            W.pad(pos);
+        if (RNULL(L, ka.reg))
+            continue;
+        bits |= 1ULL << j;
+        const int64_t v = L.R[ka.reg];
+        if (num)
+        {
+            char *p = buf + pos;
+            switch (ka.width)
+            {
+                case 1: *(int8_t *)p = (int8_t)v; pos += 1; break;
+                case 2: *(int16_t *)p = (int16_t)v; pos += 2; break;
+                case 4: *(int32_t *)p = (int32_t)v; pos += 4; break;
+                case 8: *(int64_t *)p = v; pos += 8; break;
+                default:
+                {
+                    if (ka.domain == XD_NUM)
+                    {
+                        pos += num_reg_varlena_write(L, ka.reg, (uint8_t *)p);
+                        infomask |= HEAP_HASVARWIDTH;
+                        break;
+                    }
+                    const uint32_t len = (uint32_t)L.R[ka.reg + 1];
+                    const uint8_t *s = (const uint8_t *)(uintptr_t)v;
+                    *(uint32_t *)p = (len + 4) << 2;
+                    for (uint32_t i = 0; i < len; i++)
+                        p[4 + i] = s[i];
+                    pos += 4 + len;
+                    break;
+                }
+            }
+            continue;
+        }
+        switch (ka.width)
+        {
+            case 1: W.put((uint8_t)v, 1); break;
+            case 2: W.put((uint16_t)v, 2); break;
+            case 4: W.put((uint32_t)v, 4); break;
+            case 8: W.put((uint64_t)v, 8); break;
+            default:
+            {
+                const uint32_t len = (uint32_t)L.R[ka.reg + 1];
+                const uint8_t *s = (const uint8_t *)(uintptr_t)v;
+                W.put((uint32_t)((len + 4) << 2), 4);
+                for (uint32_t i = 0; i < len; i++)
+                    W.put(s[i], 1);
+                break;
+            }
+        }
+        pos = W.pos;
+    }
+    pos += ROWID_SIZE;
+    if (num)
+        *(uint32_t *)(buf + pos - ROWID_SIZE) = rowid;
+    else
+    {
+        W.put(rowid, ROWID_SIZE);
+        W.pad(unit - (uint32_t)offsetof(kern_hashitem, t));
+    }
+    gst<uint64_t>(&hi->t.t_len, (uint64_t)pos | (uint64_t)hash << 32);
+    gst<uint64_t>(buf + 8, (uint64_t)(nattrs & HEAP_NATTS_MASK) << 16 | (uint64_t)infomask << 32 |
+                           (uint64_t)(uint8_t)(t_hoff + MINIMAL_TUPLE_OFFSET) << 48 | bits << 56);
+    for (uint32_t k = 16; k < t_hoff; k += 8)
+        gst<uint64_t>(buf + k, k == 16 ? bits >> 8 : 0);
 }
 
 /* A row may use the LDS table when every aggregate argument is non-NULL and
@@ -3162,17 +3405,61 @@ bloom_build_range(kern_data_store *ik, uint64_t *words, uint32_t mask, uint64_t 
  * kds->usage runs past them (the host recomputes it from the row index
  * before it grows the buffer).  The row id is taken after the space, so the
  * row index has no hole either (the reference instead locks nitems around
- * both, cuda_gpupreagg.cu:1141-1168). */
+ * both, cuda_gpupreagg.cu:1141-1168).  The lanes of a wave that allocate
+ * together take their space and row ids with one atomic each (a million
+ * inserted groups otherwise queue two million atomics on one cache line);
+ * their reservations follow each other in lane order, so the prefix rule
+ * holds among them too. */
 __device__ __forceinline__ kern_hashitem *
 gb_alloc(kern_data_store *kds, uint32_t unit, uint32_t *p_rowid)
 {
-    const uint64_t fixed = KDS_HEAD_LENGTH(kds) + 8ULL * kds->hash_nslots;
-    const unsigned long long end =
-        atomicAdd((unsigned long long *)&kds->usage, (unsigned long long)unit) + unit;
-    if (fixed + end + 8ULL * (end / XPU_L1_CACHELINE_SZ) > kds->length)
-        return nullptr;
-    *p_rowid = atomicAdd(&kds->nitems, 1U);
-    return hashitem_at(kds, end);
+    const uint64_t below = (1ULL << __lane_id()) - 1;
+    const uint64_t self = (uint64_t)(uintptr_t)kds;
+    kern_hashitem *hi = nullptr;
+    bool waiting = true;
+    /* one round per buffer: kds_final, then the overflow table */
+    while (waiting)
+    {
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)self);
+        const uint32_t up = __builtin_amdgcn_readfirstlane((uint32_t)(self >> 32));
+        if (self == ((uint64_t)up << 32 | lo))
+        {
+            /* units are multiples of 128: sums over the lanes bit by bit */
+            const uint32_t u = unit / XPU_L1_CACHELINE_SZ;
+            uint64_t before = 0, all = 0;
+            for (int b = 0; __ballot((u >> b) != 0) != 0; b++)
+            {
+                const uint64_t m = __ballot((u >> b) & 1);
+                before += (uint64_t)__popcll(m & below) << b;
+                all += (uint64_t)__popcll(m) << b;
+            }
+            const int leader = __ffsll((unsigned long long)__ballot(1)) - 1;
+            uint64_t base = 0;
+            if ((int)__lane_id() == leader)
+                base = atomicAdd((unsigned long long *)&kds->usage,
+                                 (unsigned long long)(all * XPU_L1_CACHELINE_SZ));
+            base = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)base, leader) |
+                   (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(base >> 32), leader) << 32;
+            const uint64_t end = base + before * XPU_L1_CACHELINE_SZ + unit;
+            const uint64_t fixed = KDS_HEAD_LENGTH(kds) + 8ULL * kds->hash_nslots;
+            const bool fits = fixed + end + 8ULL * (end / XPU_L1_CACHELINE_SZ) <= kds->length;
+            const uint64_t m = __ballot(fits);
+            if (m != 0)
+            {
+                uint32_t r0 = 0;
+                if ((int)__lane_id() == leader)
+                    r0 = atomicAdd(&kds->nitems, (uint32_t)__popcll(m));
+                r0 = (uint32_t)__builtin_amdgcn_readlane((int)r0, leader);
+                if (fits)
+                {
+                    *p_rowid = r0 + (uint32_t)__popcll(m & below);
+                    hi = hashitem_at(kds, end);
+                }
+            }
+            waiting = false;
+        }
+    }
+    return hi;
 }
 
 /* merges the partial states of group tuple src into group tuple dst (both
@@ -3336,19 +3623,30 @@ gb_tuple_keys(cplan *P, Lane &L, const kern_tupitem *t)
     }
 }
 
-/* the group tuple of the key registers on the chain from head, or null */
+/* the group tuple of the key registers on the chain from head, or null.  All
+ * lanes stay in the walk until the wave's last chain ends, so the result is a
+ * per-lane register that no divergent loop exit carries. */
 __device__ __forceinline__ kern_hashitem *
 gb_chain_find(cplan *P, const Lane &L, kern_data_store *kds, uint64_t head, uint32_t hash)
 {
-    for (uint64_t off = head; off != 0; )
+    uint64_t off = head, found = 0;
+    while (wave_any(off != 0))
     {
-        kern_hashitem *hi = hashitem_at(kds, off);
-        const uint32_t h2 = __hip_atomic_load(&hi->t.hash, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (h2 == hash && gb_keys_match(P, L, &hi->t))
-            return hi;
-        off = __hip_atomic_load(&hi->next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (off != 0)
+        {
+            kern_hashitem *hi = hashitem_at(kds, off);
+            const uint64_t next = gld<uint64_t>(&hi->next);
+            if (gld<uint32_t>(&hi->t.hash) == hash && gb_keys_match(P, L, &hi->t))
+            {
+                found = off;
+                off = 0;
+            }
+            else
+                off = next;
+        }
     }
-    return nullptr;
+    asm volatile("" : "+v"(found));
+    return found ? hashitem_at(kds, found) : nullptr;
 }
 
 /* Find-or-insert the group of the key registers of every pending lane and
@@ -3385,32 +3683,27 @@ gb_global(cplan *P, Lane &L, kern_data_store *kds_final, uint32_t hash, bool pen
         }
         return;
     }
+    const bool num = gb_num_keys(P);
+    const bool init_merged = gb_init_merged(P);
     kern_data_store *kds = kds_final;
     uint64_t *slot = (uint64_t *)((char *)kds + KDS_HEAD_LENGTH(kds)) + (hash % kds->hash_nslots);
     while (wave_any(pending))
     {
         if (pending)
         {
-            /* Slots and the fields of published group tuples are read with
-             * relaxed device-coherent loads: the inserting lane writes a tuple
-             * into a fresh 128-byte unit no other XCD has cached and publishes
-             * it with a release store, so no per-row acquire (an L2
-             * invalidate on CDNA) is needed on the lookup path. */
+            /* the slot and the published group tuples on its chain are read
+             * device-coherently (gld), without a fence */
             uint64_t head = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             kern_hashitem *found = nullptr;
             if (head != XGB_LOCKED_SLOT)
             {
                 found = gb_chain_find(P, L, kds, head, hash);
-                if (!found)
+                if (!found && num)
                 {
-                    /* A miss is confirmed after an acquire: the relaxed
-                     * walk reads a group's key bytes with plain loads, which
-                     * may hit a stale copy of its unit in this XCD's L2
-                     * (the unit was zero-filled before the group was
-                     * inserted from another XCD), and a false miss would
-                     * insert the group twice.  The acquire pairs with the
-                     * release that published `head`; misses are rare next
-                     * to hits, so lookups stay fence-free. */
+                    /* the plain reads of a numeric key may hit a stale copy
+                     * of its unit in this XCD's L2: a miss is confirmed
+                     * after an acquire, which pairs with the release that
+                     * published `head` */
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
                     found = gb_chain_find(P, L, kds, head, hash);
                 }
@@ -3441,15 +3734,28 @@ gb_global(cplan *P, Lane &L, kern_data_store *kds_final, uint32_t hash, bool pen
                     }
                     else
                     {
-                        gb_tuple_write(P, L, hi, unit, hash, rowid, head);
+                        gb_tuple_write(P, L, hi, unit, hash, rowid, head, T, lds_slot, src,
+                                       init_merged);
                         uint64_t *rowidx = (uint64_t *)((char *)kds + KDS_HEAD_LENGTH(kds)) +
                                            kds->hash_nslots;
                         rowidx[rowid] = (uint64_t)((char *)kds + kds->length - (char *)&hi->t);
-                        __hip_atomic_store(slot, (uint64_t)((char *)kds + kds->length - (char *)hi),
-                                           __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                        const uint64_t item = (uint64_t)((char *)kds + kds->length - (char *)hi);
+                        if (num)
+                            __hip_atomic_store(slot, item, __ATOMIC_RELEASE,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                        else
+                        {
+                            /* the tuple's stores have reached the point of
+                             * coherence when they complete */
+                            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                            gst<uint64_t>(slot, item);
+                        }
                         if (kds != kds_final)
                             ctl->final_ovf = 1U;
-                        found = hi;
+                        if (init_merged)
+                            pending = false;
+                        else
+                            found = hi;
                     }
                 }
             }
@@ -3668,7 +3974,7 @@ lds_update(cplan *P, const Lane &L, LdsTable &T, int slot)
     }
 }
 
-__device__ void
+__device__ __forceinline__ void
 lds_init(cplan *P, LdsTable &T)
 {
     for (uint32_t i = threadIdx.x; i < T.n; i += blockDim.x)
@@ -3714,8 +4020,13 @@ lds_init(cplan *P, LdsTable &T)
     }
 }
 
-/* merges every entry of the block's LDS table into kds_final (after a
- * barrier that ends all updates of the table) */
+/* Merges every entry of the block's LDS table into kds_final (called by the
+ * whole block, after a barrier that ends all updates of the table).  The
+ * occupied entries are gathered so that a wave merges 64 at a time, by as
+ * many waves as they fill: the partition tables of the dump merge hold a few
+ * dozen groups among their thousands of entries, and one full wave shares
+ * one space and one row-id reservation where eight sparse waves queued one
+ * each per group. */
 template <int NR>
 __device__ __forceinline__ void
 lds_flush(cplan *P, LdsTable &T, kern_data_store *kds_final, xpu_task_ctl *ctl,
@@ -3731,27 +4042,65 @@ lds_flush(cplan *P, LdsTable &T, kern_data_store *kds_final, xpu_task_ctl *ctl,
     for (int i = 0; i < NR; i++)
         L.R[i] = 0;
     L.R[XP_REG_TRUE] = 1;
-    uint32_t nflush = 0;
+    uint32_t total = 0;
     for (uint32_t base = 0; base < T.n; base += blockDim.x)
     {
-        uint32_t h = base + threadIdx.x;
-        bool pending = false;
-        uint32_t hash = 0;
-        if (h < T.n)
-        {
-            unsigned long long key = T.keys[h];
-            if (key != XLDS_EMPTY_KEY)
-            {
-                gb_unpack_key(P, L, key);
-                hash = gb_hash_regs(P, L);
-                pending = true;
-                nflush++;
-            }
-        }
-        gb_global(P, L, kds_final, hash, pending, &T, pending ? (int)h : -1, ctl, kds_ovf);
+        const uint32_t h = base + threadIdx.x;
+        total += (uint32_t)__syncthreads_count(h < T.n && T.keys[h] != XLDS_EMPTY_KEY);
     }
-    if (nflush)
-        atomicAdd((unsigned long long *)&ctl->global_merges, (unsigned long long)nflush);
+    if (total == 0)
+        return;
+    if (threadIdx.x == 0)
+        atomicAdd((unsigned long long *)&ctl->global_merges, (unsigned long long)total);
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t nfull = (total + 63) / 64;
+    const uint32_t nw = nfull < (blockDim.x >> 6) ? nfull : (blockDim.x >> 6);
+    if (wid >= nw)
+        return;
+    const uint32_t lane = __lane_id();
+    const uint32_t lo = (uint32_t)((uint64_t)T.n * wid / nw);
+    const uint32_t hi = (uint32_t)((uint64_t)T.n * (wid + 1) / nw);
+    /* lane i < nq holds a gathered entry */
+    uint32_t queue = 0, nq = 0;
+    for (uint32_t base = lo; base < hi || nq > 0; base += 64)
+    {
+        const uint32_t h = base + lane;
+        const bool occ = base < hi && h < hi && T.keys[h] != XLDS_EMPTY_KEY;
+        const uint64_t m = __ballot(occ);
+        const uint32_t k = (uint32_t)__popcll(m);
+        /* entry of rank r goes to lane (nq + r) % 64: the lanes past 63 wrap
+         * around to the next batch */
+        const uint32_t to = (nq + (uint32_t)__popcll(m & ((1ULL << lane) - 1))) & 63;
+        /* lanes without an entry send theirs to the lanes that are left */
+        const uint32_t free_to = (nq + k + (uint32_t)__popcll(~m & ((1ULL << lane) - 1))) & 63;
+        const uint32_t moved =
+            (uint32_t)__builtin_amdgcn_ds_permute((int)((occ ? to : free_to) << 2), (int)h);
+        const uint32_t end = nq + k;
+        const uint32_t fresh = (lane - nq) & 63;        /* < k: this lane got an entry */
+        const bool last = base + 64 >= hi;
+        if (end >= 64 || last)
+        {
+            /* a full batch, or what is left: lanes nq.. take the new entries
+             * of this batch, those that wrapped stay queued */
+            const uint32_t slot = lane < nq ? queue : moved;
+            const bool pending = lane < (end < 64 ? end : 64);
+            uint32_t hash = 0;
+            if (pending)
+            {
+                gb_unpack_key(P, L, T.keys[slot]);
+                hash = gb_hash_regs(P, L);
+            }
+            gb_global(P, L, kds_final, hash, pending, &T, pending ? (int)slot : -1, ctl, kds_ovf);
+            nq = end > 64 ? end - 64 : 0;
+            queue = moved;
+        }
+        else
+        {
+            if (fresh < k)
+                queue = moved;
+            nq = end;
+        }
+    }
 }
 
 /* ------------------------------------------------------------------
@@ -3776,8 +4125,10 @@ dump_rec_words(cplan *P)
 
 /* writes the block's table as partial-state records (entries beyond a
  * partition's capacity merge into kds_final directly) */
+/* inlined: as a called function it costs the scan kernel 132 registers, more
+ * than a 1024-thread block can have */
 template <int NR>
-__device__ void
+__device__ __forceinline__ void
 lds_dump(cplan *P, LdsTable &T, const xpu_kparams &kp)
 {
     __shared__ uint32_t s_cnt[XP_DUMP_MAXPARTS];
@@ -3922,37 +4273,39 @@ dump_merge_body(cplan *P, const xpu_kparams &kp)
                                                     __HIP_MEMORY_SCOPE_AGENT);
         const uint64_t n = reserved < kp.dump_cap ? reserved : kp.dump_cap;
         const uint64_t *recs = kp.dump + (uint64_t)part * kp.dump_cap * rw;
-        for (uint64_t i0 = 0; i0 < n; i0 += blockDim.x)
+        /* A table that fills up is merged once every record that found its
+         * group in it is folded; the records that found no room (a bit per
+         * record in their thread's register) go on with the emptied table.
+         * So a group merges into kds_final once per 64 records a thread
+         * holds, however many groups a partition has: a key that found no
+         * room never finds any until the table is emptied. */
+        for (uint64_t c0 = 0; c0 < n; c0 += 64ULL * blockDim.x)
         {
-            const uint64_t i = i0 + threadIdx.x;
-            const uint64_t *rec = recs + i * rw;
-            bool fail = false;
-            if (i < n)
+            const uint64_t c1 = c0 + 64ULL * blockDim.x < n ? c0 + 64ULL * blockDim.x : n;
+            uint64_t left = ~0ULL;
+            for (;;)
             {
-                int slot = lds_probe(T, rec[0]);
-                if (slot >= 0)
-                    lds_merge_entry(P, T, slot, rec);
-                else
-                    fail = true;
-            }
-            while (__syncthreads_or(fail))
-            {
-                /* the table is full: merge it, start over, then fold the
-                 * records that found no room (each round places at least
-                 * one of them in the emptied table) */
+                uint64_t again = 0;
+                for (uint32_t k = 0; c0 + (uint64_t)k * blockDim.x < c1; k++)
+                {
+                    const uint64_t i = c0 + (uint64_t)k * blockDim.x + threadIdx.x;
+                    if (i < c1 && ((left >> k) & 1))
+                    {
+                        const uint64_t *rec = recs + i * rw;
+                        const int slot = lds_probe(T, rec[0]);
+                        if (slot >= 0)
+                            lds_merge_entry(P, T, slot, rec);
+                        else
+                            again |= 1ULL << k;
+                    }
+                }
+                if (!__syncthreads_or(again != 0))
+                    break;
                 lds_flush<NR>(P, T, kp.kds_out, kp.ctl, kp.kds_ovf);
                 __syncthreads();
                 lds_init(P, T);
                 __syncthreads();
-                if (fail)
-                {
-                    int slot = lds_probe(T, rec[0]);
-                    if (slot >= 0)
-                    {
-                        lds_merge_entry(P, T, slot, rec);
-                        fail = false;
-                    }
-                }
+                left = again;
             }
         }
         __syncthreads();

@@ -1070,6 +1070,8 @@ struct JitFns
     hipFunction_t   swrite = nullptr;       /* scan + projection: write pass */
     hipFunction_t   screen = nullptr;       /* multi-pass joins: screen pass */
     hipFunction_t   probe[XP_MAX_DEPTH + 1] = {};  /* multi-pass joins: pass of depth d */
+    uint32_t        max_block = XP_AGG_BLOCK_MAX;   /* threads per block that main and
+                                                       batch can be launched with */
 };
 std::mutex g_mod_lock;
 std::map<const std::vector<char> *, JitFns> g_mods;
@@ -1128,6 +1130,21 @@ jit_function(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
             snprintf(name, sizeof(name), "xpu_jit_probe_kernel_%u", d);
             if (!hip_ok(hipModuleGetFunction(&f.probe[d], mod, name), eb, "hipModuleGetFunction"))
                 return nullptr;
+        }
+    }
+    /* a SIMD's 512 registers hold the four waves it gets of a 1024-thread
+     * block only at 128 registers a wave: a kernel that was given more (the
+     * compilers of different ROCm releases differ) runs narrower blocks */
+    if (kind == XJ_SCAN_AGG)
+    {
+        for (hipFunction_t fn : {f.main, f.batch})
+        {
+            int regs = 0;
+            if (!hip_ok(hipFuncGetAttribute(&regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, fn), eb,
+                        "hipFuncGetAttribute"))
+                return nullptr;
+            if (regs > 128)
+                f.max_block = XP_BLOCK_MAX;
         }
     }
     return &(g_mods[code] = f);
@@ -1389,8 +1406,9 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
             return ERRCODE_DEVICE_ERROR;
     }
     /* the interpreter's kernels take blocks of up to XP_BLOCK_MAX threads */
-    if (!jf && block > XP_BLOCK_MAX)
-        block = XP_BLOCK_MAX;
+    const uint32_t max_block = jf ? jf->max_block : XP_BLOCK_MAX;
+    if (block > max_block)
+        block = max_block;
     /* a projection without joins runs over wave tiles of 64*XP_PROJ_RPT rows */
     const bool sproj = !preagg && P->nrels == 0 && jf && jf->scount;
     uint32_t rows_per_tile = sproj ? 64 * XP_PROJ_RPT : block * rpt;
@@ -2983,8 +3001,8 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
             return ERRCODE_DEVICE_ERROR;
     }
     /* the interpreter's kernels take blocks of up to XP_BLOCK_MAX threads */
-    if (!jf && block > XP_BLOCK_MAX)
-        block = XP_BLOCK_MAX;
+    if (block > (jf ? jf->max_block : XP_BLOCK_MAX))
+        block = jf ? jf->max_block : XP_BLOCK_MAX;
 
     const bool replay = (flags & XPUHIP_BATCH_GRAPH) && b->gexec && b->sig == sig;
     if (!replay)

@@ -1,0 +1,54 @@
+"""Insertion of groups into kds_final: group counts around the 64 entries a
+wave merges at a time and around one LDS table, and text keys whose bytes
+end at every offset of the 8-byte words their tuple is written in.  Groups
+equal the oracle's, each once, with row ids 0..n-1."""
+import numpy as np
+import pytest
+
+from pgstrom import codegen as cg, kds, workloads as W, abi
+from helpers import assert_groups_equal, run_gpu_groupby, run_oracle_groupby
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(cols, keys, jit):
+    plan = cg.Plan([(c.name, c.typname) for c in cols])
+    kv = [plan.scan_var(k) for k in keys]
+    tlist = W.preagg_tlist(plan, kv[0], plan.scan_var("v"), plan.scan_var("w"), plan.scan_var("x"))
+    tlist += [(abi.KAGG_ACTION__VREF, k, (n, k.typname)) for n, k in zip(keys[1:], kv[1:])]
+    plan.set_groupby(tlist)
+    blob = plan.build(final_nrows=5000)
+    src = kds.build_arrow_kds(cols)
+    fin = run_gpu_groupby(blob, [src, src], tuning=dict(jit=jit))
+    exp = run_oracle_groupby(blob, [src, src])
+    got = assert_groups_equal(fin, exp, [a for a, _, _ in tlist])
+    assert sorted(r for _, r in kds.parse_row_kds(fin)) == list(range(len(got)))
+
+
+def _args(n, r):
+    return [kds.Column("v", "int8", r.integers(-1000, 1_000_000, size=n, dtype=np.int64)),
+            kds.Column("w", "float8", r.random(n)),
+            kds.Column("x", "int4", r.integers(-2**31, 2**31 - 1, size=n, dtype=np.int32))]
+
+
+@pytest.mark.parametrize("ngroups", [1, 63, 64, 65, 127, 129, 512, 3993, 9001])
+def test_group_counts(gpu, jit, ngroups):
+    r = np.random.default_rng(ngroups)
+    n = 3 * ngroups + 5
+    key = np.concatenate([np.arange(ngroups), r.integers(0, ngroups, size=n - ngroups)])
+    _check([kds.Column("key", "int4", key.astype(np.int32))] + _args(n, r), ["key"], jit)
+
+
+@pytest.mark.parametrize("second", [None, "int2"])
+def test_text_keys_of_every_length(gpu, jit, second):
+    r = np.random.default_rng(5)
+    n = 6000
+    texts = [bytes(97 + (i + j) % 26 for j in range(i % 41)) for i in range(300)]
+    null = r.random(n) < 0.05
+    cols = [kds.Column("key", "text", [texts[i] for i in r.integers(0, 300, size=n)], null)]
+    keys = ["key"]
+    if second:
+        cols.append(kds.Column("k2", "int2", r.integers(-2, 3, size=n).astype(np.int16),
+                               r.random(n) < 0.1))
+        keys.append("k2")
+    _check(cols + _args(n, r), keys, jit)
