@@ -176,6 +176,9 @@ xpu_jit_source(const xplan *P, int kind, int param)
         s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
              "xpu_jit_batch_spill_kernel(xpu_kparams kp)\n{\n";
         append(s, "    batch_spill_body<%d, JitProg>((cplan *)xjit_plan, kp);\n}\n", nr);
+        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
+             "xpu_jit_batch_merge_kernel(xpu_kparams kp)\n{\n";
+        append(s, "    batch_merge_body<%d, JitProg>((cplan *)xjit_plan, kp);\n}\n", nr);
     }
     return s;
 }

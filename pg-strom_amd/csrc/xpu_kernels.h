@@ -151,6 +151,9 @@ typedef struct
     const int64_t *params;              /* XO_PARAM values */
     uint64_t   *spill;                  /* the fragment's spill region */
     uint64_t    spill_cap;              /* records */
+    uint64_t   *dump;                   /* the fragment's partial-state records */
+    uint64_t    dump_cap;               /* records per partition */
+    uint64_t   *dump_next;              /* [dump_nparts] records reserved */
     uint64_t    param_nulls;
     uint32_t    nrows;
     uint32_t    __pad;
@@ -165,17 +168,16 @@ typedef struct
     uint32_t    __pad;
 } xbatch_item;
 
-/* a hash partition of a slice of one fragment's spill records (pass 2) */
+/* a slice of one fragment's spill records (pass 2) */
 typedef struct
 {
     uint32_t    frag;
-    uint16_t    part;
-    uint16_t    nparts;
+    uint32_t    __pad;
     uint64_t    lo;
     uint64_t    hi;
 } xbatch_sitem;
 
-#define XBATCH_SPILL_SLICE  (2ULL << 20)    /* spill records per pass-2 item */
+#define XBATCH_SPILL_SLICE  (64ULL << 10)   /* spill records per pass-2 item */
 
 typedef struct
 {
@@ -261,8 +263,9 @@ int xpu_launch_final_merge_ovf(const xplan *plan, int nregs, kern_data_store *kd
                                xpu_task_ctl *ctl, void *stream);
 /* the spill setup kernel of a batch alone (for specialized pass kernels) */
 int xpu_launch_batch_setup(const xpu_kparams *kp, void *stream);
-/* batched fragments: pass 1, spill setup, pass 2 (all stream-ordered) */
-int xpu_launch_batch(const xpu_kparams *kp, int nregs, int rpt, int grid, int block,
+/* batched fragments: pass 1, spill setup, pass 2, dump merge over mgrid
+ * blocks (all stream-ordered) */
+int xpu_launch_batch(const xpu_kparams *kp, int nregs, int rpt, int grid, int mgrid, int block,
                      size_t lds_bytes, void *stream);
 /* second pass over the spill records of a scan + group-by launch */
 int xpu_launch_spill_agg(const xpu_kparams *kp, int nregs, int grid, int block,

@@ -66,6 +66,13 @@ xpu_batch_spill_kernel(xpu_kparams kp)
     batch_spill_body<NR, Interp>((cplan *)(uintptr_t)kp.plan, kp);
 }
 
+template <int NR>
+__global__ void __launch_bounds__(XP_BLOCK_MAX)
+xpu_batch_merge_kernel(xpu_kparams kp)
+{
+    batch_merge_body<NR, Interp>((cplan *)(uintptr_t)kp.plan, kp);
+}
+
 /* ------------------------------------------------------------------
  * helper kernels
  * ------------------------------------------------------------------ */
@@ -163,7 +170,8 @@ xpu_launch_scan_agg(const xpu_kparams *kp, int nregs, int rpt, int grid, int blo
 
 template <int NR>
 static void
-launch_batch(const xpu_kparams *kp, int rpt, int grid, int block, size_t lds, hipStream_t s)
+launch_batch(const xpu_kparams *kp, int rpt, int grid, int mgrid, int block, size_t lds,
+             hipStream_t s)
 {
     if (rpt >= 4)
         hipLaunchKernelGGL((xpu_batch_agg_kernel<NR, 4>), dim3(grid), dim3(block), lds, s, *kp);
@@ -173,6 +181,8 @@ launch_batch(const xpu_kparams *kp, int rpt, int grid, int block, size_t lds, hi
         hipLaunchKernelGGL((xpu_batch_agg_kernel<NR, 1>), dim3(grid), dim3(block), lds, s, *kp);
     hipLaunchKernelGGL(xpu_batch_spill_setup_kernel, dim3(1), dim3(64), 0, s, *kp);
     hipLaunchKernelGGL((xpu_batch_spill_kernel<NR>), dim3(grid), dim3(block), lds, s, *kp);
+    if (mgrid > 0)
+        hipLaunchKernelGGL((xpu_batch_merge_kernel<NR>), dim3(mgrid), dim3(block), lds, s, *kp);
 }
 
 extern "C" int
@@ -183,13 +193,13 @@ xpu_launch_batch_setup(const xpu_kparams *kp, void *stream)
 }
 
 extern "C" int
-xpu_launch_batch(const xpu_kparams *kp, int nregs, int rpt, int grid, int block,
+xpu_launch_batch(const xpu_kparams *kp, int nregs, int rpt, int grid, int mgrid, int block,
                  size_t lds_bytes, void *stream)
 {
     if (nregs <= XP_NREGS_SMALL)
-        launch_batch<XP_NREGS_SMALL>(kp, rpt, grid, block, lds_bytes, (hipStream_t)stream);
+        launch_batch<XP_NREGS_SMALL>(kp, rpt, grid, mgrid, block, lds_bytes, (hipStream_t)stream);
     else
-        launch_batch<XP_NREGS>(kp, rpt, grid, block, lds_bytes, (hipStream_t)stream);
+        launch_batch<XP_NREGS>(kp, rpt, grid, mgrid, block, lds_bytes, (hipStream_t)stream);
     return (int)hipGetLastError();
 }
 

@@ -1063,6 +1063,7 @@ struct JitFns
     hipFunction_t   spill = nullptr;        /* spill pass (scan + group-by) */
     hipFunction_t   batch = nullptr;        /* batched pass 1 */
     hipFunction_t   batch_spill = nullptr;  /* batched pass 2 */
+    hipFunction_t   batch_merge = nullptr;  /* batched pass 3 */
     hipFunction_t   dump = nullptr;         /* partial-state dump merge */
     hipFunction_t   count = nullptr;        /* projection count pass */
     hipFunction_t   write = nullptr;        /* projection write pass */
@@ -1103,6 +1104,8 @@ jit_function(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
          !hip_ok(hipModuleGetFunction(&f.batch, mod, "xpu_jit_batch_kernel"), eb,
                  "hipModuleGetFunction") ||
          !hip_ok(hipModuleGetFunction(&f.batch_spill, mod, "xpu_jit_batch_spill_kernel"), eb,
+                 "hipModuleGetFunction") ||
+         !hip_ok(hipModuleGetFunction(&f.batch_merge, mod, "xpu_jit_batch_merge_kernel"), eb,
                  "hipModuleGetFunction") ||
          !hip_ok(hipModuleGetFunction(&f.dump, mod, "xpu_jit_dump_kernel"), eb,
                  "hipModuleGetFunction")))
@@ -2841,6 +2844,8 @@ struct BatchScratch
     xpu_task_ctl *h_ctl = nullptr;      size_t hctl_cap = 0;
     uint32_t   *d_ticket = nullptr;     size_t ticket_cap = 0;
     uint64_t   *d_spill = nullptr;      size_t spill_cap = 0;
+    uint64_t   *d_dump = nullptr;       size_t dump_cap = 0;
+    uint64_t   *d_dump_next = nullptr;  size_t dump_next_cap = 0;
     std::vector<uint64_t> sig;
     hipGraph_t  graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -2848,8 +2853,11 @@ struct BatchScratch
 std::mutex g_batch_lock;
 BatchScratch g_batch;
 
-#define XBATCH_MAX_SITEMS   16384
 #define XBATCH_SPILL_BYTES  (8ULL << 30)    /* spill buffer of a batch at most */
+#define XBATCH_DUMP_BYTES   (4ULL << 30)    /* partial-state records of a batch at most */
+/* dump merge work (fragments x partitions) of a batch: eight blocks' worth
+ * per CU, and at least eight partitions a fragment */
+#define XBATCH_MERGE_ITEMS  2048
 
 void
 batch_drop_graph(BatchScratch *b)
@@ -2980,6 +2988,39 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
         }
     }
 
+    /* spill slices: every fragment ends with a partial one */
+    const uint32_t nsitems = (uint32_t)(spill_recs / XBATCH_SPILL_SLICE) + ntasks;
+
+    /* partial-state records: a table for each work item of the fragment and
+     * its spilled rows, an eighth more for uneven partitions; entries past a
+     * partition's capacity merge into kds_final directly */
+    uint32_t nparts = 0;
+    const uint64_t rw = 1 + P->lds_n64 + (1 + P->lds_n32 + 1) / 2;
+    std::vector<uint64_t> dcaps(ntasks, 0);
+    uint64_t dump_recs = 0;
+    if (spill)
+    {
+        nparts = std::min<uint32_t>(XP_DUMP_MAXPARTS,
+                                    std::max<uint32_t>(8, XBATCH_MERGE_ITEMS / ntasks));
+        for (uint32_t f = 0; f < ntasks; f++)
+        {
+            const uint64_t nitems_f = ((uint64_t)tasks[f].nitems + item_rows - 1) / item_rows;
+            const uint64_t n = std::min<uint64_t>(nitems_f * lds_nents + caps[f], tasks[f].nitems);
+            dcaps[f] = n / nparts * 9 / 8 + 256;
+            dump_recs += dcaps[f] * nparts;
+        }
+        if (dump_recs * rw * 8 > XBATCH_DUMP_BYTES)
+        {
+            const double k = (double)XBATCH_DUMP_BYTES / (double)(dump_recs * rw * 8);
+            dump_recs = 0;
+            for (uint32_t f = 0; f < ntasks; f++)
+            {
+                dcaps[f] = (uint64_t)(dcaps[f] * k);
+                dump_recs += dcaps[f] * nparts;
+            }
+        }
+    }
+
     std::vector<uint64_t> sig;
     sig.push_back(ntasks);
     sig.push_back(flags);
@@ -3009,10 +3050,13 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     {
         if (!batch_grow(b, (char **)&b->d_frags, &b->frags_cap, sizeof(xbatch_frag) * ntasks, eb) ||
             !batch_grow(b, (char **)&b->d_items, &b->items_cap, sizeof(xbatch_item) * items.size(), eb) ||
-            !batch_grow(b, (char **)&b->d_sitems, &b->sitems_cap, sizeof(xbatch_sitem) * XBATCH_MAX_SITEMS, eb) ||
+            !batch_grow(b, (char **)&b->d_sitems, &b->sitems_cap, sizeof(xbatch_sitem) * nsitems, eb) ||
             !batch_grow(b, (char **)&b->d_ctl, &b->ctl_cap, sizeof(xpu_task_ctl) * ntasks, eb) ||
             !batch_grow(b, (char **)&b->d_ticket, &b->ticket_cap, 64, eb) ||
-            (spill && !batch_grow(b, (char **)&b->d_spill, &b->spill_cap, spill_recs * rec, eb)))
+            (spill && !batch_grow(b, (char **)&b->d_spill, &b->spill_cap, spill_recs * rec, eb)) ||
+            (spill && !batch_grow(b, (char **)&b->d_dump, &b->dump_cap, dump_recs * rw * 8, eb)) ||
+            (spill && !batch_grow(b, (char **)&b->d_dump_next, &b->dump_next_cap,
+                                  8ULL * nparts * ntasks, eb)))
             return ERRCODE_DEVICE_ERROR;
         if (b->hctl_cap < sizeof(xpu_task_ctl) * ntasks)
         {
@@ -3026,7 +3070,7 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
             b->hctl_cap = sizeof(xpu_task_ctl) * ntasks;
         }
         std::vector<xbatch_frag> frags(ntasks);
-        uint64_t off = 0;
+        uint64_t off = 0, doff = 0;
         for (uint32_t f = 0; f < ntasks; f++)
         {
             xpuhip_session *s = tasks[f].sess;
@@ -3040,8 +3084,12 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
             fr.param_nulls = s->comp.param_nulls;
             fr.spill = spill ? b->d_spill + off * (rec / 8) : nullptr;
             fr.spill_cap = caps[f];
+            fr.dump = spill ? b->d_dump + doff * rw : nullptr;
+            fr.dump_cap = dcaps[f];
+            fr.dump_next = spill ? b->d_dump_next + (uint64_t)f * nparts : nullptr;
             fr.nrows = tasks[f].nitems;
             off += caps[f];
+            doff += dcaps[f] * nparts;
         }
         if (!hip_ok(hipMemcpy(b->d_frags, frags.data(), sizeof(xbatch_frag) * ntasks,
                               hipMemcpyHostToDevice), eb, "hipMemcpy") ||
@@ -3062,16 +3110,21 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     kp.batch_ticket = b->d_ticket;
     kp.batch_nfrags = ntasks;
     kp.batch_nitems = (uint32_t)items.size();
-    kp.batch_nsitems_cap = XBATCH_MAX_SITEMS;
+    kp.batch_nsitems_cap = nsitems;
+    kp.dump_nparts = nparts;
+    const uint32_t mgrid = std::min<uint32_t>(nparts * ntasks, 4 * (uint32_t)g_dev.ncu);
 
-    /* the launch sequence: clear control blocks and tickets, pass 1, spill
-     * setup, pass 2 (no memset nodes: capturable) */
+    /* the launch sequence: clear control blocks, tickets and dump counters,
+     * pass 1, spill setup, pass 2, dump merge (no memset nodes: capturable) */
     auto enqueue = [&]() -> int {
         int rc = xpu_launch_fill(b->d_ctl, 0, sizeof(xpu_task_ctl) * ntasks / 8, b->stream);
         if (!rc)
             rc = xpu_launch_fill(b->d_ticket, 0, 8, b->stream);
+        if (!rc && nparts)
+            rc = xpu_launch_fill(b->d_dump_next, 0, (size_t)nparts * ntasks, b->stream);
         if (rc)
             return rc;
+        const uint32_t sblock = block < XP_BLOCK_MAX ? block : XP_BLOCK_MAX;
         if (jf)
         {
             void *args[] = {&kp};
@@ -3080,12 +3133,14 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
             if (!rc)
                 rc = xpu_launch_batch_setup(&kp, b->stream);
             if (!rc)
-                rc = (int)hipModuleLaunchKernel(jf->batch_spill, grid, 1, 1,
-                                                block < XP_BLOCK_MAX ? block : XP_BLOCK_MAX, 1, 1,
+                rc = (int)hipModuleLaunchKernel(jf->batch_spill, grid, 1, 1, sblock, 1, 1,
+                                                (unsigned)lds, b->stream, args, nullptr);
+            if (!rc && mgrid)
+                rc = (int)hipModuleLaunchKernel(jf->batch_merge, mgrid, 1, 1, sblock, 1, 1,
                                                 (unsigned)lds, b->stream, args, nullptr);
             return rc;
         }
-        return xpu_launch_batch(&kp, P->nregs, (int)rpt, grid, block, lds, b->stream);
+        return xpu_launch_batch(&kp, P->nregs, (int)rpt, grid, (int)mgrid, block, lds, b->stream);
     };
 
     int rc = 0;

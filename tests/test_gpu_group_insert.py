@@ -5,7 +5,7 @@ equal the oracle's, each once, with row ids 0..n-1."""
 import numpy as np
 import pytest
 
-from pgstrom import codegen as cg, kds, workloads as W, abi
+from pgstrom import abi, codegen as cg, datagen, kds, workloads as W, xpuhip
 from helpers import assert_groups_equal, run_gpu_groupby, run_oracle_groupby
 
 pytestmark = pytest.mark.gpu
@@ -52,3 +52,49 @@ def test_text_keys_of_every_length(gpu, jit, second):
                                r.random(n) < 0.1))
         keys.append("k2")
     _check(cols + _args(n, r), keys, jit)
+
+
+@pytest.mark.parametrize("lds_nents", [64, 1024, 2000])
+def test_partitions_with_more_groups_than_a_table(gpu, jit, lds_nents):
+    """Spilled rows and dumps of 150,000 groups: a dump partition holds about
+    600 of them, fewer or more than the table it is folded in."""
+    r = np.random.default_rng(lds_nents)
+    n = 300_000
+    key = np.concatenate([np.arange(150_000), r.integers(0, 150_000, size=n - 150_000)])
+    cols = [kds.Column("key", "int4", r.permutation(key).astype(np.int32))] + _args(n, r)
+    plan = cg.Plan([(c.name, c.typname) for c in cols])
+    tlist = W.preagg_tlist(plan, *[plan.scan_var(k) for k in ("key", "v", "w", "x")])
+    plan.set_groupby(tlist)
+    blob = plan.build(final_nrows=150_000)
+    src = kds.build_arrow_kds(cols)
+    fin = run_gpu_groupby(blob, [src], tuning=dict(jit=jit, lds_nents=lds_nents))
+    assert_groups_equal(fin, run_oracle_groupby(blob, [src]), [a for a, _, _ in tlist])
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_of_uneven_fragments(gpu, jit, graph):
+    """Fragments of 1 to 200,000 rows and 1 to 10,000 groups in one launch,
+    run twice: each equals its session alone."""
+    r = np.random.default_rng(8)
+    sizes = [(1, 3), (64, 1), (4097, 9000), (70_001, 17), (200_000, 100_000)]
+    base = 200_000
+    cols = datagen.preagg_table(base)
+    cols = [kds.Column("a", "int4", r.integers(0, 1_000_000, size=base, dtype=np.int32))] + cols
+    chunk = kds.build_arrow_kds(cols)
+    hdrs = kds.window_headers(chunk, [(0, n) for n, _ in sizes], len(sizes) * 1024, 1024)
+    dev = xpuhip.DeviceBuffer(len(hdrs) + len(chunk), np.concatenate([hdrs, chunk]))
+    acts = [a for a, _, _ in W.preagg_tlist(None, cols[1], None, None, None)]
+    tasks, alone = [], []
+    for i, (n, m) in enumerate(sizes):
+        blob = W.fragment_query(cols, k=700_000, m=m)
+        s = xpuhip.Session(blob)
+        s.set_tuning(jit=jit, lds_nents=1024)
+        tasks.append((s, dev.ptr + i * 1024, n))
+        part = kds.build_arrow_kds(datagen.take_rows(cols, np.arange(base) < n))
+        alone.append(run_oracle_groupby(blob, [part, part]))
+    for _ in range(2):
+        xpuhip.batch_exec(tasks, graph=graph)
+    for (s, _, _), exp in zip(tasks, alone):
+        assert_groups_equal(s.final(), exp, acts)
+        s.close()
+    dev.free()
