@@ -984,8 +984,21 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
 }
 
 /* a scan + group-by block merges its LDS table into kds_final once: below
- * this many rows per block the merges outweigh the rows */
+ * this many rows per block the merges outweigh the rows.  Where the tables
+ * leave as partial-state dumps a group merges once however many blocks hold
+ * it, and what a block costs is its table's set-up and its dump counters:
+ * two wave tiles of the widest shape are enough (60,001 rows with NULLs, 30
+ * blocks instead of 2: scan pass 1.78 -> 0.25 ms) */
 #define XPU_MIN_ROWS_PER_BLOCK  (32ULL << 10)
+#define XPU_MIN_ROWS_PER_DUMP   (2ULL << 10)
+
+/* spill and dump records of a scan + group-by task: room for every row while
+ * that takes no more than this.  A table of many groups sends most rows past
+ * the LDS tables, and each row beyond the records costs a find-or-insert in
+ * kds_final with its own atomics (6M rows over 1M groups:
+ * scan pass 11.7 ms with room for a quarter, 0.26 ms with room for all) */
+#define XPU_SPILL_BYTES         (512ULL << 20)
+#define XPU_DUMP_BYTES          (512ULL << 20)
 
 /* XPUHIP_JIT_AUTO specializes chunks of at least this many rows */
 #define XPUHIP_JIT_AUTO_ROWS    1000000ULL
@@ -1421,17 +1434,17 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
      * (6M rows: 0.38 ms against 0.49 ms; 50M rows: 2.6 ms against 3.9 ms) */
     uint32_t bpc = t.blocks_per_cu ? t.blocks_per_cu : (sproj && nrows > (4ULL << 20) ? 4 : 2);
     uint32_t grid = (uint32_t)g_dev.ncu * bpc;
-    if (scan_agg)
+    uint32_t lds_nents = (preagg && P->lds_fast) ? t.lds_nents : 0;
+    const bool spill = scan_agg && P->spill_ok && lds_nents > 0;
+    if (scan_agg && lds_nents > 0)
     {
-        /* a block's LDS table costs an init and a merge into kds_final: give
-         * each block at least XPU_MIN_ROWS_PER_BLOCK rows */
-        uint64_t by_rows = (nrows + XPU_MIN_ROWS_PER_BLOCK - 1) / XPU_MIN_ROWS_PER_BLOCK;
+        const uint64_t min_rows = spill ? XPU_MIN_ROWS_PER_DUMP : XPU_MIN_ROWS_PER_BLOCK;
+        uint64_t by_rows = (nrows + min_rows - 1) / min_rows;
         if (grid > by_rows)
             grid = (uint32_t)by_rows;
     }
     if (grid > ntiles)
         grid = ntiles;      /* scan_agg: a block tile is its waves' first tiles */
-    uint32_t lds_nents = (preagg && P->lds_fast) ? t.lds_nents : 0;
     size_t lds = lds_bytes_for(P, lds_nents);
     if (lds + (scan_agg ? 0 : XP_PIPELINE_STATIC_LDS) > g_dev.lds_per_block)
     {
@@ -1472,13 +1485,16 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
         }
         kp.prefilter = (preagg && P->nrels > 0) ? 1 : 0;
     }
-    /* spill buffer of a scan + group-by: room for a quarter of the rows (at
-     * least 1M records); rows beyond it merge into kds_final directly */
-    const bool spill = scan_agg && P->spill_ok && lds_nents > 0;
+    /* spill buffer of a scan + group-by: room for every row (and the records
+     * each wave reserves ahead) up to XPU_SPILL_BYTES, and for a quarter of
+     * the rows above; rows beyond it merge into kds_final directly */
     if (spill)
     {
         uint64_t rec = 8ULL * (1 + P->spill_nregs);
-        uint64_t nrec = nrows / 4 > (1ULL << 20) ? nrows / 4 : (1ULL << 20);
+        const uint64_t all = nrows + (uint64_t)grid * (block / 64) * XSPILL_CHUNK;
+        /* a table of a few entries folds next to nothing before it dumps */
+        const uint64_t room = lds_nents >= 1024 ? XPU_SPILL_BYTES / rec : 1ULL << 20;
+        const uint64_t nrec = std::min<uint64_t>(all, std::max<uint64_t>(nrows / 4, room));
         if (!grow((char **)&x->d_spill, &x->spill_cap, nrec * rec, eb))
             return ERRCODE_DEVICE_ERROR;
         kp.spill = x->d_spill;
@@ -1489,8 +1505,13 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
         uint32_t nparts = (uint32_t)g_dev.ncu < XP_DUMP_MAXPARTS ? (uint32_t)g_dev.ncu : XP_DUMP_MAXPARTS;
         uint64_t rw = 1 + P->lds_n64 + (1 + P->lds_n32 + 1) / 2;
         /* one table per block from the scan pass plus the spill pass's
-         * dumps of full tables: room for eight tables per block */
-        uint64_t per_part = (8ULL * grid * lds_nents) / nparts + 4096;
+         * dumps of full tables: a record for every spilled row at most, and
+         * beyond XPU_DUMP_BYTES room for eight tables per block; an eighth
+         * more for uneven partitions */
+        const uint64_t ndump = std::min<uint64_t>((uint64_t)grid * lds_nents + std::min<uint64_t>(nrec, nrows),
+                                                  std::max<uint64_t>(8ULL * grid * lds_nents,
+                                                                     XPU_DUMP_BYTES / (8 * rw)));
+        uint64_t per_part = ndump / nparts * 9 / 8 + 1024;
         if (!grow((char **)&x->d_dump, &x->dump_cap, per_part * nparts * rw * 8, eb) ||
             !grow((char **)&x->d_dump_next, &x->dump_next_cap, 8ULL * XP_DUMP_MAXPARTS, eb))
             return ERRCODE_DEVICE_ERROR;
