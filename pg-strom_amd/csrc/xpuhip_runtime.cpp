@@ -133,6 +133,101 @@ ensure_device(kern_errorbuf *eb)
     return 0;
 }
 
+/* Device buffers of closed sessions, kept for the next ones: a backend opens
+ * a session per query, and giving its buffers (a 1 GiB kds_final and its
+ * overflow table among them) back to the driver makes the next hipMalloc of
+ * that size wait until the driver has cleared the freed memory (a 2M-row
+ * star query opened and closed in a row: 42 ms a query, 1.9 ms with the
+ * buffers kept).  Buffers are reused
+ * by rounded size; at most DEVPOOL_KEEP_BYTES stay idle, all go back when an
+ * allocation fails or at xpuhip_shutdown.  A buffer is given back only after
+ * the work that used it has completed (every entry point waits for its own). */
+#define DEVPOOL_KEEP_BYTES      (8ULL << 30)
+#define DEVPOOL_KEEP_COUNT      1024
+
+struct DevPool
+{
+    std::mutex  lock;
+    std::map<void *, size_t> live;                  /* buffer -> rounded size */
+    std::multimap<size_t, void *> idle;
+    size_t      idle_bytes = 0;
+
+    /* at most an eighth more than asked for */
+    static size_t
+    round_up(size_t n)
+    {
+        size_t step = 256;
+        while (step * 16 <= n)
+            step <<= 1;
+        return (n + step - 1) & ~(step - 1);
+    }
+    hipError_t
+    alloc(void **p, size_t n)
+    {
+        const size_t sz = round_up(n);
+        {
+            std::lock_guard<std::mutex> g(lock);
+            auto it = idle.find(sz);
+            if (it != idle.end())
+            {
+                *p = it->second;
+                idle.erase(it);
+                idle_bytes -= sz;
+                live[*p] = sz;
+                return hipSuccess;
+            }
+        }
+        hipError_t rc = hipMalloc(p, sz);
+        if (rc == hipErrorOutOfMemory)
+        {
+            (void)hipGetLastError();
+            trim();
+            rc = hipMalloc(p, sz);
+        }
+        if (rc == hipSuccess)
+        {
+            std::lock_guard<std::mutex> g(lock);
+            live[*p] = sz;
+        }
+        return rc;
+    }
+    void
+    free(void *p)
+    {
+        if (!p)
+            return;
+        {
+            std::lock_guard<std::mutex> g(lock);
+            auto it = live.find(p);
+            if (it != live.end())
+            {
+                const size_t sz = it->second;
+                live.erase(it);
+                if (idle_bytes + sz <= DEVPOOL_KEEP_BYTES && idle.size() < DEVPOOL_KEEP_COUNT)
+                {
+                    idle.emplace(sz, p);
+                    idle_bytes += sz;
+                    return;
+                }
+            }
+        }
+        (void)hipFree(p);
+    }
+    void
+    trim()
+    {
+        std::multimap<size_t, void *> gone;
+        {
+            std::lock_guard<std::mutex> g(lock);
+            gone.swap(idle);
+            idle_bytes = 0;
+        }
+        for (auto &e : gone)
+            (void)hipFree(e.second);
+    }
+};
+DevPool     g_pool;
+
 /* per-call device scratch: control block, look-back words, staging */
 struct Scratch
 {
@@ -166,6 +261,7 @@ struct Scratch
     size_t      hmeta_cap = 0;
     xheap_status *h_hstat = nullptr;    /* pinned */
     hipEvent_t  evh0 = nullptr, evh1 = nullptr;
+    char       *h_final = nullptr;      /* pinned: a small final's write-back */
     std::vector<char> h_tiles_head;
     std::vector<xheap_col> h_hcols;
 };
@@ -205,6 +301,7 @@ scratch_destroy(Scratch *s)
     if (s->d_tiles) (void)hipFree(s->d_tiles);
     if (s->d_hmeta) (void)hipFree(s->d_hmeta);
     if (s->h_hstat) (void)hipHostFree(s->h_hstat);
+    if (s->h_final) (void)hipHostFree(s->h_final);
     if (s->evh0) (void)hipEventDestroy(s->evh0);
     if (s->evh1) (void)hipEventDestroy(s->evh1);
     if (s->ev0) (void)hipEventDestroy(s->ev0);
@@ -234,9 +331,22 @@ grow(char **p, size_t *cap, size_t need, kern_errorbuf *eb)
 
 bool xpuhip_tuned_shape(const xplan *P, xpuhip_tuning *t);
 
+struct JitFns;
+
+/* what the sessions of one plan shape share for the life of the process */
+struct PlanShared
+{
+    std::mutex      lock;
+    /* the specialized kernels by (kind, param), found once: their key in the
+     * code cache is the whole kernel source, which takes 0.15 ms to write out */
+    std::map<int, const JitFns *> jit;
+};
+static PlanShared *plan_shared(const xplan *P);
+
 struct xpuhip_session
 {
     xpu_compiled    comp;
+    PlanShared     *shared = nullptr;
     xplan          *d_plan = nullptr;
     char           *d_const_pool = nullptr;
     kern_data_store *d_kds_dst_head = nullptr;
@@ -274,6 +384,9 @@ struct xpuhip_session
     std::vector<Scratch *> pool;
     uint64_t        ntasks = 0;
 };
+
+/* bytes of the pinned write-back staging of small finals */
+#define XPU_FINAL_STAGE         (4ULL << 20)
 
 /* Pinned inner buffers (gpu_service.c:2099-2196): the KDS_FORMAT_HASH
  * buffer that the projections of every session of one query_plan_id append
@@ -594,6 +707,7 @@ xpuhip_shutdown(void)
     std::lock_guard<std::mutex> g(g_dev_lock);
     if (g_dev.ready)
         (void)hipDeviceSynchronize();
+    g_pool.trim();
     g_dev.ready = false;
 }
 
@@ -671,10 +785,11 @@ xpuhip_session_open(const kern_session_info *session, size_t length,
         if (xpuhip_tuned_shape(&s->comp.plan, &tt))
             s->tuning = tt;
     }
+    s->shared = plan_shared(&s->comp.plan);
     /* plan and constants */
     size_t pool_len = s->comp.const_pool.size() ? s->comp.const_pool.size() : 8;
-    if (!hip_ok(hipMalloc((void **)&s->d_const_pool, pool_len), eb, "hipMalloc") ||
-        !hip_ok(hipMalloc((void **)&s->d_plan, sizeof(xplan)), eb, "hipMalloc"))
+    if (!hip_ok(g_pool.alloc((void **)&s->d_const_pool, pool_len), eb, "hipMalloc") ||
+        !hip_ok(g_pool.alloc((void **)&s->d_plan, sizeof(xplan)), eb, "hipMalloc"))
     {
         xpuhip_session_close(s);
         return ERRCODE_DEVICE_ERROR;
@@ -689,7 +804,7 @@ xpuhip_session_open(const kern_session_info *session, size_t length,
     s->comp.plan.const_pool = (uint64_t)(uintptr_t)s->d_const_pool;
     {
         size_t np = s->comp.params.size() ? s->comp.params.size() : 1;
-        if (!hip_ok(hipMalloc((void **)&s->d_params, 8 * np), eb, "hipMalloc") ||
+        if (!hip_ok(g_pool.alloc((void **)&s->d_params, 8 * np), eb, "hipMalloc") ||
             (!s->comp.params.empty() &&
              !hip_ok(hipMemcpy(s->d_params, s->comp.params.data(), 8 * s->comp.params.size(),
                                hipMemcpyHostToDevice), eb, "hipMemcpy")))
@@ -699,7 +814,7 @@ xpuhip_session_open(const kern_session_info *session, size_t length,
         }
     }
     if (!s->comp.xids.empty() &&
-        (!hip_ok(hipMalloc((void **)&s->d_xids, 4 * s->comp.xids.size()), eb, "hipMalloc") ||
+        (!hip_ok(g_pool.alloc((void **)&s->d_xids, 4 * s->comp.xids.size()), eb, "hipMalloc") ||
          !hip_ok(hipMemcpy(s->d_xids, s->comp.xids.data(), 4 * s->comp.xids.size(),
                            hipMemcpyHostToDevice), eb, "hipMemcpy")))
     {
@@ -708,7 +823,7 @@ xpuhip_session_open(const kern_session_info *session, size_t length,
     }
     if (!s->comp.kds_dst_head.empty())
     {
-        if (!hip_ok(hipMalloc((void **)&s->d_kds_dst_head, s->comp.kds_dst_head.size()), eb, "hipMalloc") ||
+        if (!hip_ok(g_pool.alloc((void **)&s->d_kds_dst_head, s->comp.kds_dst_head.size()), eb, "hipMalloc") ||
             !hip_ok(hipMemcpy(s->d_kds_dst_head, s->comp.kds_dst_head.data(), s->comp.kds_dst_head.size(),
                               hipMemcpyHostToDevice), eb, "hipMemcpy"))
         {
@@ -725,7 +840,7 @@ xpuhip_session_open(const kern_session_info *session, size_t length,
             len = need + (64ULL << 20);
         len &= ~(uint64_t)(XPU_L1_CACHELINE_SZ - 1);
         s->final_length = len;
-        if (!hip_ok(hipMalloc((void **)&s->d_kds_final, len), eb, "hipMalloc(kds_final)") ||
+        if (!hip_ok(g_pool.alloc((void **)&s->d_kds_final, len), eb, "hipMalloc(kds_final)") ||
             (rc = init_kds_final(s, eb)) != 0)
         {
             xpuhip_session_close(s);
@@ -741,7 +856,7 @@ xpuhip_session_open(const kern_session_info *session, size_t length,
         fh->nitems = 0;
         fh->usage = 0;
         fh->length &= ~(uint64_t)(XPU_MAXIMUM_ALIGNOF - 1);
-        if (!hip_ok(hipMalloc((void **)&s->d_kds_fallback, fh->length), eb, "hipMalloc(kds_fallback)") ||
+        if (!hip_ok(g_pool.alloc((void **)&s->d_kds_fallback, fh->length), eb, "hipMalloc(kds_fallback)") ||
             !hip_ok(hipMemcpy(s->d_kds_fallback, img.data(), img.size(), hipMemcpyHostToDevice), eb,
                     "hipMemcpy"))
         {
@@ -768,7 +883,7 @@ xpuhip_session_open(const kern_session_info *session, size_t length,
                 len = need;
             len = (len + XPU_L1_CACHELINE_SZ - 1) & ~(uint64_t)(XPU_L1_CACHELINE_SZ - 1);
             s->final_length = len;
-            if (!hip_ok(hipMalloc((void **)&s->d_kds_final, len), eb, "hipMalloc(pinned buffer)") ||
+            if (!hip_ok(g_pool.alloc((void **)&s->d_kds_final, len), eb, "hipMalloc(pinned buffer)") ||
                 (rc = init_kds_final(s, eb)) != 0)
             {
                 xpuhip_session_close(s);
@@ -839,10 +954,10 @@ attach_pinned(xpuhip_session *s, uint32_t d, uint64_t plan_id, uint64_t *nitems_
     h->length = length;
     h->hash_nslots = nslots;
     if (s->d_inner_own[d])
-        (void)hipFree(s->d_inner_own[d]);
+        g_pool.free(s->d_inner_own[d]);
     s->d_inner_own[d] = nullptr;
     char *dst = nullptr;
-    if (!hip_ok(hipMalloc((void **)&dst, length), eb, "hipMalloc(inner buffer)"))
+    if (!hip_ok(g_pool.alloc((void **)&dst, length), eb, "hipMalloc(inner buffer)"))
         return ERRCODE_DEVICE_ERROR;
     s->d_inner_own[d] = dst;
     if (!hip_ok(hipMemcpy(dst, head.data(), hl, hipMemcpyHostToDevice), eb, "hipMemcpy") ||
@@ -904,9 +1019,9 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
         }
     }
     if (s->d_kmrels)
-        (void)hipFree(s->d_kmrels);
+        g_pool.free(s->d_kmrels);
     s->d_kmrels = nullptr;
-    if (!hip_ok(hipMalloc((void **)&s->d_kmrels, length), eb, "hipMalloc(kmrels)") ||
+    if (!hip_ok(g_pool.alloc((void **)&s->d_kmrels, length), eb, "hipMalloc(kmrels)") ||
         !hip_ok(hipMemcpy(s->d_kmrels, kmrels, length, hipMemcpyHostToDevice), eb, "hipMemcpy(kmrels)"))
         return ERRCODE_DEVICE_ERROR;
     uint64_t d_nitems[XP_MAX_DEPTH + 1] = {}, d_nslots[XP_MAX_DEPTH + 1] = {};
@@ -928,10 +1043,11 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
         }
         P->depth[d].left_outer = ch->left_outer ? 1 : 0;
     }
+    s->shared = plan_shared(P);     /* LEFT OUTER is part of the plan's shape */
     /* Bloom filters: 16 to 32 bits per item in 64-bit words (a power of two,
      * at most 2^23 words), built from the hash chains just copied */
     if (s->d_bloom)
-        (void)hipFree(s->d_bloom);
+        g_pool.free(s->d_bloom);
     s->d_bloom = nullptr;
     uint64_t nwords = 0;
     for (uint32_t d = 1; d <= P->nrels; d++)
@@ -952,7 +1068,7 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
         const uint64_t w1 = (uint64_t)s->bloom_mask[1] + 1;
         s->bloom_lds_words = (uint32_t)(w1 < XQ_SCREEN_LDS_WORDS ? w1 : XQ_SCREEN_LDS_WORDS);
         s->bloom_lds_off = nwords + ndup;
-        if (!hip_ok(hipMalloc((void **)&s->d_bloom, 8 * (nwords + ndup + s->bloom_lds_words)), eb,
+        if (!hip_ok(g_pool.alloc((void **)&s->d_bloom, 8 * (nwords + ndup + s->bloom_lds_words)), eb,
                     "hipMalloc(bloom)") ||
             !hip_ok((hipError_t)xpu_launch_fill(s->d_bloom, 0, nwords + ndup, nullptr), eb, "bloom fill"))
             return ERRCODE_DEVICE_ERROR;
@@ -1069,6 +1185,8 @@ join_pass_sizes(const xplan *P, const uint32_t *maxdup, uint64_t nrows, uint32_t
     return true;
 }
 
+}   /* namespace */
+
 /* code objects of specialized kernels loaded into this process's device */
 struct JitFns
 {
@@ -1087,11 +1205,14 @@ struct JitFns
     uint32_t        max_block = XP_AGG_BLOCK_MAX;   /* threads per block that main and
                                                        batch can be launched with */
 };
+
+namespace {
+
 std::mutex g_mod_lock;
 std::map<const std::vector<char> *, JitFns> g_mods;
 
 const JitFns *
-jit_function(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
+jit_load(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
 {
     std::string log;
     const std::vector<char> *code = xpu_jit_code(&s->comp.plan, kind, param, &log);
@@ -1166,6 +1287,26 @@ jit_function(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
     return &(g_mods[code] = f);
 }
 
+const JitFns *
+jit_function(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
+{
+    const int key = kind * 16 + param;
+    PlanShared *sh = s->shared;
+    {
+        std::lock_guard<std::mutex> g(sh->lock);
+        auto it = sh->jit.find(key);
+        if (it != sh->jit.end())
+            return it->second;
+    }
+    const JitFns *f = jit_load(s, kind, param, eb);
+    if (f)
+    {
+        std::lock_guard<std::mutex> g(sh->lock);
+        sh->jit[key] = f;
+    }
+    return f;
+}
+
 }   /* namespace */
 
 /* ------------------------------------------------------------------
@@ -1220,7 +1361,7 @@ ensure_ovf(xpuhip_session *s, uint64_t nrows, kern_errorbuf *eb)
         return 0;
     if (s->d_kds_ovf)
     {
-        (void)hipFree(s->d_kds_ovf);
+        g_pool.free(s->d_kds_ovf);
         s->d_kds_ovf = nullptr;
         s->ovf_length = 0;
     }
@@ -1228,7 +1369,7 @@ ensure_ovf(xpuhip_session *s, uint64_t nrows, kern_errorbuf *eb)
     const uint32_t nslots = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(want / 512, 1024),
                                                          UINT32_MAX / 2);
     std::vector<char> img = ovf_head(s, want, nslots);
-    if (!hip_ok(hipMalloc((void **)&s->d_kds_ovf, want), eb, "hipMalloc(group-by overflow table)"))
+    if (!hip_ok(g_pool.alloc((void **)&s->d_kds_ovf, want), eb, "hipMalloc(group-by overflow table)"))
     {
         s->d_kds_ovf = nullptr;
         return ERRCODE_DEVICE_ERROR;
@@ -1237,7 +1378,7 @@ ensure_ovf(xpuhip_session *s, uint64_t nrows, kern_errorbuf *eb)
         xpu_launch_fill((char *)s->d_kds_ovf + img.size(), 0, nslots, nullptr) != 0 ||
         !hip_ok(hipDeviceSynchronize(), eb, "overflow table init"))
     {
-        (void)hipFree(s->d_kds_ovf);
+        g_pool.free(s->d_kds_ovf);
         s->d_kds_ovf = nullptr;
         return ERRCODE_DEVICE_ERROR;
     }
@@ -1292,7 +1433,7 @@ final_grow_merge(xpuhip_session *s, Scratch *x, kern_errorbuf *eb)
         new_len = need;
     new_len = (new_len + XPU_L1_CACHELINE_SZ - 1) & ~(uint64_t)(XPU_L1_CACHELINE_SZ - 1);
     kern_data_store *d_new = nullptr;
-    if (!hip_ok(hipMalloc((void **)&d_new, new_len), eb, "hipMalloc(kds_final)"))
+    if (!hip_ok(g_pool.alloc((void **)&d_new, new_len), eb, "hipMalloc(kds_final)"))
         return ERRCODE_DEVICE_ERROR;
     /* head, slots and row index stay; the tuples keep their distance from
      * the tail, so chains and row index stay valid */
@@ -1332,10 +1473,10 @@ final_grow_merge(xpuhip_session *s, Scratch *x, kern_errorbuf *eb)
     if (rc != 0)
     {
         (void)hipStreamSynchronize(x->stream);
-        (void)hipFree(d_new);
+        g_pool.free(d_new);
         return rc;
     }
-    (void)hipFree(s->d_kds_final);
+    g_pool.free(s->d_kds_final);
     s->d_kds_final = d_new;
     s->final_length = new_len;
     t_last_stats.final_grows++;
@@ -2419,10 +2560,10 @@ sort_final(xpuhip_session *s, uint32_t n, uint32_t nout, const uint64_t *d_ridx,
     if (need > s->sort_cap)
     {
         if (s->d_sort)
-            (void)hipFree(s->d_sort);
+            g_pool.free(s->d_sort);
         s->d_sort = nullptr;
         s->sort_cap = 0;
-        if (!hip_ok(hipMalloc((void **)&s->d_sort, need), eb, "hipMalloc(sort)"))
+        if (!hip_ok(g_pool.alloc((void **)&s->d_sort, need), eb, "hipMalloc(sort)"))
             return -1;
         s->sort_cap = need;
     }
@@ -2636,6 +2777,32 @@ xpuhip_task_final(xpuhip_session *s, kern_data_store *out, size_t length,
     h->nitems = (uint32_t)nout;
     h->usage = usage;
     memcpy(out, hbuf.data(), head_len);
+    if (8 * nout + usage <= XPU_FINAL_STAGE)
+    {
+        /* small finals (10,000 groups of five aggregates: 1.4 MB) through
+         * pinned memory with one wait */
+        Scratch *x = scratch_get(s, eb);
+        if (!x)
+            return -1;
+        const bool ok =
+            (x->h_final || hip_ok(hipHostMalloc((void **)&x->h_final, XPU_FINAL_STAGE,
+                                                hipHostMallocDefault), eb, "hipHostMalloc")) &&
+            hip_ok(hipMemcpyAsync(x->h_final, d_ridx, 8 * nout, hipMemcpyDeviceToHost, x->stream), eb,
+                   "hipMemcpyAsync") &&
+            (usage == 0 ||
+             hip_ok(hipMemcpyAsync(x->h_final + 8 * nout, d_tail, usage, hipMemcpyDeviceToHost,
+                                   x->stream), eb, "hipMemcpyAsync")) &&
+            hip_ok(hipStreamSynchronize(x->stream), eb, "hipStreamSynchronize");
+        if (ok)
+        {
+            memcpy((char *)out + head_len, x->h_final, 8 * nout);
+            memcpy((char *)out + need - usage, x->h_final + 8 * nout, usage);
+        }
+        scratch_put(s, x);
+        if (!ok)
+            return -1;
+        return (int64_t)need;
+    }
     if (!hip_ok(hipMemcpy((char *)out + head_len, d_ridx,
                           8 * nout, hipMemcpyDeviceToHost), eb, "hipMemcpy") ||
         (usage > 0 &&
@@ -2710,9 +2877,9 @@ xpuhip_session_close(xpuhip_session *s)
     for (Scratch *x : s->pool)
         scratch_retire(x);
     s->pool.clear();
-    if (s->d_plan) (void)hipFree(s->d_plan);
-    if (s->d_const_pool) (void)hipFree(s->d_const_pool);
-    if (s->d_kds_dst_head) (void)hipFree(s->d_kds_dst_head);
+    if (s->d_plan) g_pool.free(s->d_plan);
+    if (s->d_const_pool) g_pool.free(s->d_const_pool);
+    if (s->d_kds_dst_head) g_pool.free(s->d_kds_dst_head);
     if (s->pinned)
     {
         /* the plan's last session frees its pinned buffer */
@@ -2720,7 +2887,7 @@ xpuhip_session_close(xpuhip_session *s)
         if (--s->pinned->refs == 0)
         {
             (void)hipDeviceSynchronize();
-            (void)hipFree(s->pinned->d_kds);
+            g_pool.free(s->pinned->d_kds);
             g_pinned.erase(s->pinned->plan_id);
             delete s->pinned;
         }
@@ -2728,17 +2895,17 @@ xpuhip_session_close(xpuhip_session *s)
         s->d_kds_final = nullptr;
     }
     else if (s->d_kds_final)
-        (void)hipFree(s->d_kds_final);
-    if (s->d_kds_ovf) (void)hipFree(s->d_kds_ovf);
-    if (s->d_kds_fallback) (void)hipFree(s->d_kds_fallback);
-    if (s->d_kmrels) (void)hipFree(s->d_kmrels);
-    if (s->d_bloom) (void)hipFree(s->d_bloom);
-    if (s->d_params) (void)hipFree(s->d_params);
-    if (s->d_xids) (void)hipFree(s->d_xids);
-    if (s->d_sort) (void)hipFree(s->d_sort);
+        g_pool.free(s->d_kds_final);
+    if (s->d_kds_ovf) g_pool.free(s->d_kds_ovf);
+    if (s->d_kds_fallback) g_pool.free(s->d_kds_fallback);
+    if (s->d_kmrels) g_pool.free(s->d_kmrels);
+    if (s->d_bloom) g_pool.free(s->d_bloom);
+    if (s->d_params) g_pool.free(s->d_params);
+    if (s->d_xids) g_pool.free(s->d_xids);
+    if (s->d_sort) g_pool.free(s->d_sort);
     if (s->d_sort_stage) (void)hipFree(s->d_sort_stage);
     for (int d = 0; d <= XP_MAX_DEPTH; d++)
-        if (s->d_inner_own[d]) (void)hipFree(s->d_inner_own[d]);
+        if (s->d_inner_own[d]) g_pool.free(s->d_inner_own[d]);
     delete s;
 }
 
@@ -3048,9 +3215,16 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     sig.push_back(((uint64_t)block << 32) | rpt);
     sig.push_back(((uint64_t)grid << 32) | lds_nents);
     sig.push_back(t.jit);
+    sig.push_back((uint64_t)(uintptr_t)s0->shared);
+    sig.push_back((uint64_t)(uintptr_t)s0->d_plan);
     for (uint32_t f = 0; f < ntasks; f++)
     {
-        sig.push_back((uint64_t)(uintptr_t)tasks[f].sess);
+        /* what the captured launch reads of the session: a later session may
+         * have the address of a closed one, or its kds_final may have grown */
+        sig.push_back((uint64_t)(uintptr_t)tasks[f].sess->d_kds_final);
+        sig.push_back((uint64_t)(uintptr_t)tasks[f].sess->d_params);
+        sig.push_back((uint64_t)(uintptr_t)tasks[f].sess->d_const_pool);
+        sig.push_back(tasks[f].sess->comp.param_nulls);
         sig.push_back((uint64_t)(uintptr_t)tasks[f].d_kds_src);
         sig.push_back(tasks[f].nitems);
     }
@@ -3274,6 +3448,21 @@ shape_key(const xplan *P)
     x.const_pool = 0;
     return std::string((const char *)&x, offsetof(xplan, ops) + sizeof(xop) * x.nops);
 }
+
+}   /* namespace */
+
+static PlanShared *
+plan_shared(const xplan *P)
+{
+    static std::map<std::string, std::unique_ptr<PlanShared>> shapes;
+    std::lock_guard<std::mutex> g(g_tune_lock);
+    auto &slot = shapes[shape_key(P)];
+    if (!slot)
+        slot.reset(new PlanShared());
+    return slot.get();
+}
+
+namespace {
 
 /* candidate launch shapes for a session's task kind */
 std::vector<xpuhip_tuning>
