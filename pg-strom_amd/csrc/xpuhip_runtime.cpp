@@ -1570,11 +1570,15 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
     const bool sproj = !preagg && P->nrels == 0 && jf && jf->scount;
     uint32_t rows_per_tile = sproj ? 64 * XP_PROJ_RPT : block * rpt;
     uint32_t ntiles = (uint32_t)((nrows + rows_per_tile - 1) / rows_per_tile);
-    /* wave-tile projections: two blocks per CU for chunks of up to 4M rows
-     * (1M-row scan: 0.12 ms against 0.14 ms with four), four above
-     * (6M rows: 0.38 ms against 0.49 ms; 50M rows: 2.6 ms against 3.9 ms) */
-    uint32_t bpc = t.blocks_per_cu ? t.blocks_per_cu : (sproj && nrows > (4ULL << 20) ? 4 : 2);
+    /* wave-tile projections: up to 16 blocks per CU, and no more waves than
+     * tiles.  Both passes wait for dependent loads (text offsets, then their
+     * bytes), so waves in flight count: 24M rows take 1.08 ms with two blocks
+     * per CU, 0.66 with four, 0.61 with sixteen; 1M rows 0.050 ms with two
+     * tiles a wave, 0.038 with one, 0.066 with blocks left over */
+    uint32_t bpc = t.blocks_per_cu ? t.blocks_per_cu : (sproj ? 16 : 2);
     uint32_t grid = (uint32_t)g_dev.ncu * bpc;
+    if (sproj && grid > (ntiles + block / 64 - 1) / (block / 64))
+        grid = (ntiles + block / 64 - 1) / (block / 64);
     uint32_t lds_nents = (preagg && P->lds_fast) ? t.lds_nents : 0;
     const bool spill = scan_agg && P->spill_ok && lds_nents > 0;
     if (scan_agg && lds_nents > 0)
