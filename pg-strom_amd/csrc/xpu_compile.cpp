@@ -1376,6 +1376,38 @@ layout_state_size(int action)
     return -1;
 }
 
+/* the op that loads a chunk column into register r, through moves; false if
+ * r is computed otherwise or written more than once */
+bool
+key_column_op(const std::vector<xop> &ops, int r, uint16_t *p_op)
+{
+    for (int step = 0; step < 4; step++)
+    {
+        int at = -1;
+        for (size_t i = 0; i < ops.size(); i++)
+        {
+            if (ops[i].dst != r || ops[i].op == XO_NOP || ops[i].op == XO_KILL ||
+                ops[i].op == XO_TXTCHK)
+                continue;
+            if (at >= 0)
+                return false;
+            at = (int)i;
+        }
+        if (at < 0)
+            return false;
+        const xop &o = ops[at];
+        if (o.op == XO_LDCOL || o.op == XO_LDCOL_VAR)
+        {
+            *p_op = (uint16_t)at;
+            return true;
+        }
+        if (o.op != XO_MOV && o.op != XO_MOV2)
+            return false;
+        r = o.a;
+    }
+    return false;
+}
+
 /* fields an action keeps in the LDS partial table, besides the entry's row
  * count (rows that reach the table have every argument non-NULL and every
  * FILTER true, so count(*), count(x) and the n of sums and averages are all
@@ -1694,7 +1726,7 @@ xpu_compile_session(const kern_session_info *s, size_t length, xpu_compiled *out
         uint32_t off = 0;
         bool seen_key = false;
         int nkeys = 0, key_bits = 0;
-        bool lds_ok = true;
+        bool lds_ok = true, text_key = false;
         int lds_n64 = 0, lds_n32 = 0;
         for (int j = 0; j < nattrs; j++)
         {
@@ -1737,8 +1769,10 @@ xpu_compile_session(const kern_session_info *s, size_t length, xpu_compiled *out
                 ka->width = (ka->domain == XD_TEXT || ka->domain == XD_NUM) ? -1 : type_width(t);
                 if (ka->width > 0 && cm->attlen != ka->width)
                     FAIL("grouping key width differs from the kds_final column");
-                if (ka->width < 0)
+                if (ka->domain == XD_NUM)
                     lds_ok = false;
+                else if (ka->width < 0)
+                    text_key = true;
                 else
                 {
                     P->key_bits[nkeys] = 8 * ka->width;
@@ -1780,7 +1814,17 @@ xpu_compile_session(const kern_session_info *s, size_t length, xpu_compiled *out
         P->nkeys = nkeys;
         P->gb_states_end = off;
         P->gb_t_hoff = XPU_MAXALIGN(KERN_TUPITEM_T_BITS_OFFSET + XPU_BITMAPLEN(nattrs));
-        P->lds_fast = (lds_ok && key_bits <= 63) ? 1 : 0;
+        /* text keys: by hash and row, when every key is a column of the
+         * chunk, so that a row of it stands for the key values */
+        if (lds_ok && text_key)
+        {
+            bool cols = P->nrels == 0;
+            for (int k = 0; k < nkeys && cols; k++)
+                cols = key_column_op(C.ops, P->keys[k].reg, &P->key_ld[k]);
+            P->lds_text = cols ? 1 : 0;
+            lds_ok = cols;
+        }
+        P->lds_fast = (lds_ok && (text_key || key_bits <= 63)) ? 1 : 0;
         /* registers a spill record carries: the distinct aggregate arguments */
         if (P->lds_fast && nkeys > 0)
         {

@@ -1231,6 +1231,153 @@ num_rescale(xi128 v, int scale_d, int scale_s)
     return v;
 }
 
+/* the fixed-width value (w bytes) of Arrow column col at a row; true if NULL */
+__device__ __forceinline__ bool
+ldcol_fixed(const kern_data_store *__restrict__ kds, uint32_t col, uint32_t row, int w, int domain,
+            int64_t *p_v)
+{
+    const char *kbase = (const char *)kds;
+    ccolmeta *cm = &((ckds *)(uintptr_t)kds)->colmeta[col];
+    uint64_t nm_off = cm->nullmap_offset;
+    uint64_t v_off = cm->values_offset;
+    uint64_t v_len = cm->values_length;
+    bool isnull = false;
+    if (nm_off)
+    {
+        uint32_t idx = row >> 3;
+        isnull = (idx >= cm->nullmap_length) ||
+                 !((((const uint8_t *)kbase)[nm_off + idx] >> (row & 7)) & 1);
+    }
+    /* the value is read whenever it lies inside the column, so
+     * its load does not wait for the validity bit */
+    const bool inside = (uint64_t)w * (row + 1) <= v_len;
+    int64_t v = 0;
+    if (inside)
+    {
+        const char *p = kbase + v_off + (uint64_t)w * row;
+        switch (w)
+        {
+            case 1: v = *(const int8_t *)p; break;
+            case 2: v = *(const int16_t *)p; break;
+            case 4: v = (domain == XD_F32) ? (int64_t)*(const uint32_t *)p
+                                      : (int64_t)*(const int32_t *)p; break;
+            default: v = *(const int64_t *)p; break;
+        }
+    }
+    isnull = isnull || !inside;
+    *p_v = v;
+    return isnull;
+}
+
+/* the text or binary value of Arrow column col at a row as address and
+ * length (XTEXT_RAW: a compressed or external datum); true if NULL.  A column
+ * whose type is not mappable sets *badtype. */
+__device__ __forceinline__ bool
+ldcol_var(const kern_data_store *__restrict__ kds, uint32_t col, uint32_t row, int64_t *p_ptr,
+          int64_t *p_len, bool *badtype)
+{
+    const char *kbase = (const char *)kds;
+    ccolmeta *cm = &((ckds *)(uintptr_t)kds)->colmeta[col];
+    bool isnull = false;
+    if (cm->nullmap_offset)
+    {
+        uint32_t idx = row >> 3;
+        isnull = (idx >= cm->nullmap_length) ||
+                 !((((const uint8_t *)kbase)[cm->nullmap_offset + idx] >> (row & 7)) & 1);
+    }
+    int64_t ptr = 0, len = 0;
+    if (cm->attopts.tag == XARROW_TAG_HEAPREF)
+    {
+        /* column tiles of a heap / row chunk: (offset, length)
+         * pairs into the source chunk */
+        if (8ULL * ((uint64_t)row + 1) > cm->values_length)
+            isnull = true;
+        if (!isnull)
+        {
+            uint2 pr = ((const uint2 *)(kbase + cm->values_offset))[row];
+            if (pr.y == XHEAP_LEN_EXTERNAL)
+            {
+                /* kept as it is: the offset addresses its header */
+                const uint8_t *vp = (const uint8_t *)kbase + cm->extra_offset + pr.x;
+                if ((uint64_t)pr.x + 2 > cm->extra_length ||
+                    (uint64_t)pr.x + varsize_any(vp) > cm->extra_length)
+                    isnull = true;
+                else
+                {
+                    ptr = (int64_t)(uintptr_t)vp;
+                    len = XTEXT_RAW;
+                }
+            }
+            else if ((uint64_t)pr.x + pr.y > cm->extra_length)
+                isnull = true;
+            else
+            {
+                ptr = (int64_t)((uintptr_t)kbase + cm->extra_offset + pr.x);
+                len = pr.y;
+            }
+        }
+    }
+    else if (cm->attopts.tag == ArrowType__Utf8 || cm->attopts.tag == ArrowType__Binary)
+    {
+        /* KDS_ARROW_REF_VARLENA32_DATUM (xpu_common.h:1577-1601) */
+        if (4ULL * ((uint64_t)row + 2) > cm->values_length)
+            isnull = true;
+        if (!isnull)
+        {
+            const uint32_t *off = (const uint32_t *)(kbase + cm->values_offset);
+            uint32_t o0 = off[row], o1 = off[row + 1];
+            if (o0 > o1 || o1 > cm->extra_length || o1 - o0 > XARROW_VARATT_MAX)
+                isnull = true;
+            else
+            {
+                ptr = (int64_t)(uintptr_t)(kbase + cm->extra_offset + o0);
+                len = o1 - o0;
+            }
+        }
+    }
+    else if (cm->attopts.tag == ArrowType__LargeUtf8 ||
+             cm->attopts.tag == ArrowType__LargeBinary)
+    {
+        /* KDS_ARROW_REF_VARLENA64_DATUM (xpu_common.h:1603-1626) */
+        if (8ULL * ((uint64_t)row + 2) > cm->values_length)
+            isnull = true;
+        if (!isnull)
+        {
+            const uint64_t *off = (const uint64_t *)(kbase + cm->values_offset);
+            uint64_t o0 = off[row], o1 = off[row + 1];
+            if (o0 > o1 || o1 > cm->extra_length || o1 - o0 > XARROW_VARATT_MAX)
+                isnull = true;
+            else
+            {
+                ptr = (int64_t)(uintptr_t)(kbase + cm->extra_offset + o0);
+                len = (int64_t)(o1 - o0);
+            }
+        }
+    }
+    else if (cm->attopts.tag == ArrowType__FixedSizeBinary)
+    {
+        /* KDS_ARROW_REF_SIMPLE_DATUM with the byte width
+         * (xpu_textlib.cu:30-35, xpu_common.h:1556-1573) */
+        const uint64_t w = cm->attopts.u.fixed_size_binary.byteWidth;
+        if (w * ((uint64_t)row + 1) > cm->values_length)
+            isnull = true;
+        if (!isnull)
+        {
+            ptr = (int64_t)(uintptr_t)(kbase + cm->values_offset + w * row);
+            len = (int64_t)w;
+        }
+    }
+    else
+    {
+        /* "not a mappable Arrow data type" (xpu_textlib.cu:49-51) */
+        *badtype = true;
+        isnull = true;
+    }
+    *p_ptr = ptr;
+    *p_len = len;
+    return isnull;
+}
+
 /* STAGED: the caller has loaded the columns of the plan's stage[] list into
  * their registers, so the program's XLD_STAGED loads are skipped */
 template <bool STAGED>
@@ -1249,35 +1396,8 @@ xop_exec(const xop o, Lane &L, const kern_data_store *__restrict__ kds, uint32_t
             {
                 if (STAGED && (o.imm & XLD_STAGED))
                     break;
-                ccolmeta *cm = &kmeta->colmeta[o.aux];
-                uint64_t nm_off = cm->nullmap_offset;
-                uint64_t v_off = cm->values_offset;
-                uint64_t v_len = cm->values_length;
-                int w = (int)(o.imm & XLD_WIDTH_MASK);
-                bool isnull = false;
-                if (nm_off)
-                {
-                    uint32_t idx = row >> 3;
-                    isnull = (idx >= cm->nullmap_length) ||
-                             !((((const uint8_t *)kbase)[nm_off + idx] >> (row & 7)) & 1);
-                }
-                /* the value is read whenever it lies inside the column, so
-                 * its load does not wait for the validity bit */
-                const bool inside = (uint64_t)w * (row + 1) <= v_len;
-                int64_t v = 0;
-                if (inside)
-                {
-                    const char *p = kbase + v_off + (uint64_t)w * row;
-                    switch (w)
-                    {
-                        case 1: v = *(const int8_t *)p; break;
-                        case 2: v = *(const int16_t *)p; break;
-                        case 4: v = (b == XD_F32) ? (int64_t)*(const uint32_t *)p
-                                                  : (int64_t)*(const int32_t *)p; break;
-                        default: v = *(const int64_t *)p; break;
-                    }
-                }
-                isnull = isnull || !inside;
+                int64_t v;
+                const bool isnull = ldcol_fixed(kds, o.aux, row, (int)(o.imm & XLD_WIDTH_MASK), b, &v);
                 L.R[d] = isnull ? 0 : v;
                 SETNULL(L, d, isnull);
                 break;
@@ -1300,103 +1420,11 @@ xop_exec(const xop o, Lane &L, const kern_data_store *__restrict__ kds, uint32_t
             }
             case XO_LDCOL_VAR:
             {
-                ccolmeta *cm = &kmeta->colmeta[o.aux];
-                bool isnull = false;
-                if (cm->nullmap_offset)
-                {
-                    uint32_t idx = row >> 3;
-                    isnull = (idx >= cm->nullmap_length) ||
-                             !((((const uint8_t *)kbase)[cm->nullmap_offset + idx] >> (row & 7)) & 1);
-                }
-                int64_t ptr = 0, len = 0;
-                if (cm->attopts.tag == XARROW_TAG_HEAPREF)
-                {
-                    /* column tiles of a heap / row chunk: (offset, length)
-                     * pairs into the source chunk */
-                    if (8ULL * ((uint64_t)row + 1) > cm->values_length)
-                        isnull = true;
-                    if (!isnull)
-                    {
-                        uint2 pr = ((const uint2 *)(kbase + cm->values_offset))[row];
-                        if (pr.y == XHEAP_LEN_EXTERNAL)
-                        {
-                            /* kept as it is: the offset addresses its header */
-                            const uint8_t *vp = (const uint8_t *)kbase + cm->extra_offset + pr.x;
-                            if ((uint64_t)pr.x + 2 > cm->extra_length ||
-                                (uint64_t)pr.x + varsize_any(vp) > cm->extra_length)
-                                isnull = true;
-                            else
-                            {
-                                ptr = (int64_t)(uintptr_t)vp;
-                                len = XTEXT_RAW;
-                            }
-                        }
-                        else if ((uint64_t)pr.x + pr.y > cm->extra_length)
-                            isnull = true;
-                        else
-                        {
-                            ptr = (int64_t)((uintptr_t)kbase + cm->extra_offset + pr.x);
-                            len = pr.y;
-                        }
-                    }
-                }
-                else if (cm->attopts.tag == ArrowType__Utf8 || cm->attopts.tag == ArrowType__Binary)
-                {
-                    /* KDS_ARROW_REF_VARLENA32_DATUM (xpu_common.h:1577-1601) */
-                    if (4ULL * ((uint64_t)row + 2) > cm->values_length)
-                        isnull = true;
-                    if (!isnull)
-                    {
-                        const uint32_t *off = (const uint32_t *)(kbase + cm->values_offset);
-                        uint32_t o0 = off[row], o1 = off[row + 1];
-                        if (o0 > o1 || o1 > cm->extra_length || o1 - o0 > XARROW_VARATT_MAX)
-                            isnull = true;
-                        else
-                        {
-                            ptr = (int64_t)(uintptr_t)(kbase + cm->extra_offset + o0);
-                            len = o1 - o0;
-                        }
-                    }
-                }
-                else if (cm->attopts.tag == ArrowType__LargeUtf8 ||
-                         cm->attopts.tag == ArrowType__LargeBinary)
-                {
-                    /* KDS_ARROW_REF_VARLENA64_DATUM (xpu_common.h:1603-1626) */
-                    if (8ULL * ((uint64_t)row + 2) > cm->values_length)
-                        isnull = true;
-                    if (!isnull)
-                    {
-                        const uint64_t *off = (const uint64_t *)(kbase + cm->values_offset);
-                        uint64_t o0 = off[row], o1 = off[row + 1];
-                        if (o0 > o1 || o1 > cm->extra_length || o1 - o0 > XARROW_VARATT_MAX)
-                            isnull = true;
-                        else
-                        {
-                            ptr = (int64_t)(uintptr_t)(kbase + cm->extra_offset + o0);
-                            len = (int64_t)(o1 - o0);
-                        }
-                    }
-                }
-                else if (cm->attopts.tag == ArrowType__FixedSizeBinary)
-                {
-                    /* KDS_ARROW_REF_SIMPLE_DATUM with the byte width
-                     * (xpu_textlib.cu:30-35, xpu_common.h:1556-1573) */
-                    const uint64_t w = cm->attopts.u.fixed_size_binary.byteWidth;
-                    if (w * ((uint64_t)row + 1) > cm->values_length)
-                        isnull = true;
-                    if (!isnull)
-                    {
-                        ptr = (int64_t)(uintptr_t)(kbase + cm->values_offset + w * row);
-                        len = (int64_t)w;
-                    }
-                }
-                else
-                {
-                    /* "not a mappable Arrow data type" (xpu_textlib.cu:49-51) */
-                    if (!L.err)
-                        L.err = XMSG_ARROW_TYPE + 1;
-                    isnull = true;
-                }
+                int64_t ptr, len;
+                bool badtype = false;
+                const bool isnull = ldcol_var(kds, o.aux, row, &ptr, &len, &badtype);
+                if (badtype && !L.err)
+                    L.err = XMSG_ARROW_TYPE + 1;
                 L.R[d] = ptr;
                 L.R[d + 1] = len;
                 SETNULL(L, d, isnull);
@@ -3856,47 +3884,6 @@ final_merge_ovf_body(cplan *P, kern_data_store *kds_final, const kern_data_store
     }
 }
 
-__device__ __forceinline__ uint64_t
-gb_pack_key(cplan *P, const Lane &L)
-{
-    uint64_t pk = 0;
-    int shift = 0;
-    for (int k = 0; k < (int)P->nkeys; k++)
-    {
-        int bits = P->key_bits[k];
-        int r = P->keys[k].reg;
-        uint64_t v = RNULL(L, r) ? 0 : ((uint64_t)L.R[r] & ((bits >= 64) ? ~0ULL : ((1ULL << bits) - 1)));
-        pk |= v << shift;
-        shift += bits;
-    }
-    for (int k = 0; k < (int)P->nkeys; k++)
-        pk |= (uint64_t)RNULL(L, P->keys[k].reg) << (shift + k);
-    return pk;
-}
-
-__device__ __forceinline__ void
-gb_unpack_key(cplan *P, Lane &L, uint64_t pk)
-{
-    int shift = 0;
-    for (int k = 0; k < (int)P->nkeys; k++)
-        shift += P->key_bits[k];
-    int vshift = 0;
-    for (int k = 0; k < (int)P->nkeys; k++)
-    {
-        int bits = P->key_bits[k];
-        int r = P->keys[k].reg;
-        uint64_t v = (pk >> vshift) & ((bits >= 64) ? ~0ULL : ((1ULL << bits) - 1));
-        int64_t sv;
-        if (P->keys[k].domain == XD_INT && bits < 64)
-            sv = (int64_t)(v << (64 - bits)) >> (64 - bits);     /* sign extend */
-        else
-            sv = (int64_t)v;
-        L.R[r] = sv;
-        SETNULL(L, r, (pk >> (shift + k)) & 1);
-        vshift += bits;
-    }
-}
-
 /* PG hash of the grouping keys held in registers (HashValue semantics) */
 __device__ __forceinline__ uint32_t
 gb_hash_regs(cplan *P, const Lane &L)
@@ -3925,6 +3912,146 @@ gb_hash_regs(cplan *P, const Lane &L)
     return h ^ 0xffffffffU;
 }
 
+/* Plans with text keys (P->lds_text) have no packed key values: an LDS entry,
+ * spill or dump record names its group by the keys' hash and a row of the
+ * chunk that holds them, and keys compare with that row's columns.  Without
+ * this every row found and merged its group in kds_final with its own device
+ * atomics (4M rows, 2,556 texts of 8-24 characters: 3.7 ms then, 0.60 ms
+ * in three passes now). */
+
+/* grouping key k at a row of the chunk (length of a text in *len); true if
+ * NULL */
+__device__ __forceinline__ bool
+gb_row_key(cplan *P, int k, const kern_data_store *kds, uint32_t row, int64_t *v, int64_t *len)
+{
+    const xop o = P->ops[P->key_ld[k]];
+    *len = 0;
+    if (P->keys[k].width >= 0)
+        return ldcol_fixed(kds, o.aux, row, (int)(o.imm & XLD_WIDTH_MASK), o.b, v);
+    bool badtype = false;
+    return ldcol_var(kds, o.aux, row, v, len, &badtype);
+}
+
+/* whether len bytes at p and q (any alignment) are equal; every byte is
+ * compared, with the words that hold four of them read at once */
+__device__ __forceinline__ bool
+text_same(const uint8_t *p, const uint8_t *q, uint32_t len)
+{
+    uint32_t diff = 0;
+    for (uint32_t i = 0; i < len; i += 16)
+    {
+        const uint32_t n = len - i < 16 ? len - i : 16;
+        uint64_t w[2][3];
+#pragma unroll
+        for (int side = 0; side < 2; side++)
+        {
+            const uintptr_t a = (uintptr_t)((side ? q : p) + i);
+            const uint64_t *x = (const uint64_t *)(a & ~(uintptr_t)7);
+            const uint32_t off = (uint32_t)(a & 7), sh = 8 * off;
+            const uint32_t last = (off + n - 1) >> 3;
+            uint64_t y[3];
+#pragma unroll
+            for (uint32_t j = 0; j < 3; j++)
+                y[j] = j <= last ? x[j] : 0;
+            w[side][0] = sh ? (y[0] >> sh) | (y[1] << (64 - sh)) : y[0];
+            w[side][1] = sh ? (y[1] >> sh) | (y[2] << (64 - sh)) : y[1];
+        }
+        const uint64_t m0 = n >= 8 ? ~0ULL : ~0ULL >> (64 - 8 * n);
+        const uint64_t m1 = n > 8 ? ~0ULL >> (64 - 8 * (n - 8)) : 0;
+        const uint64_t x = ((w[0][0] ^ w[1][0]) & m0) | ((w[0][1] ^ w[1][1]) & m1);
+        diff |= (uint32_t)x | (uint32_t)(x >> 32);
+    }
+    return diff == 0;
+}
+
+/* whether the rows a and b of the chunk hold the same grouping keys */
+__device__ __forceinline__ bool
+gb_rows_match(cplan *P, const kern_data_store *kds, uint32_t a, uint32_t b)
+{
+    bool same = true;
+    for (int k = 0; k < (int)P->nkeys; k++)
+    {
+        int64_t va, vb, la, lb;
+        const bool na = gb_row_key(P, k, kds, a, &va, &la);
+        const bool nb = gb_row_key(P, k, kds, b, &vb, &lb);
+        if (na || nb)
+            same = same && na == nb;
+        else if (P->keys[k].width >= 0)
+            same = same && va == vb;
+        else
+        {
+            same = same && la == lb;
+            same = same && text_same((const uint8_t *)(uintptr_t)va, (const uint8_t *)(uintptr_t)vb,
+                                     same ? (uint32_t)la : 0);
+        }
+    }
+    return same;
+}
+
+__device__ __forceinline__ uint64_t
+gb_pack_key(cplan *P, const Lane &L, uint32_t row)
+{
+    if (P->lds_text)
+        return (uint64_t)gb_hash_regs(P, L) << 32 | row;
+    uint64_t pk = 0;
+    int shift = 0;
+    for (int k = 0; k < (int)P->nkeys; k++)
+    {
+        int bits = P->key_bits[k];
+        int r = P->keys[k].reg;
+        uint64_t v = RNULL(L, r) ? 0 : ((uint64_t)L.R[r] & ((bits >= 64) ? ~0ULL : ((1ULL << bits) - 1)));
+        pk |= v << shift;
+        shift += bits;
+    }
+    for (int k = 0; k < (int)P->nkeys; k++)
+        pk |= (uint64_t)RNULL(L, P->keys[k].reg) << (shift + k);
+    return pk;
+}
+
+__device__ __forceinline__ void
+gb_unpack_key(cplan *P, Lane &L, uint64_t pk, const kern_data_store *kds)
+{
+    if (P->lds_text)
+    {
+        for (int k = 0; k < (int)P->nkeys; k++)
+        {
+            const int r = P->keys[k].reg;
+            int64_t v, len;
+            const bool isnull = gb_row_key(P, k, kds, (uint32_t)pk, &v, &len);
+            L.R[r] = isnull ? 0 : v;
+            if (P->keys[k].width < 0)
+                L.R[r + 1] = isnull ? 0 : len;
+            SETNULL(L, r, isnull);
+        }
+        return;
+    }
+    int shift = 0;
+    for (int k = 0; k < (int)P->nkeys; k++)
+        shift += P->key_bits[k];
+    int vshift = 0;
+    for (int k = 0; k < (int)P->nkeys; k++)
+    {
+        int bits = P->key_bits[k];
+        int r = P->keys[k].reg;
+        uint64_t v = (pk >> vshift) & ((bits >= 64) ? ~0ULL : ((1ULL << bits) - 1));
+        int64_t sv;
+        if (P->keys[k].domain == XD_INT && bits < 64)
+            sv = (int64_t)(v << (64 - bits)) >> (64 - bits);     /* sign extend */
+        else
+            sv = (int64_t)v;
+        L.R[r] = sv;
+        SETNULL(L, r, (pk >> (shift + k)) & 1);
+        vshift += bits;
+    }
+}
+
+/* the part of a packed key that selects its LDS slot and dump partition */
+__device__ __forceinline__ uint64_t
+gb_key_part(cplan *P, uint64_t pk)
+{
+    return P->lds_text ? pk >> 32 : pk;
+}
+
 __device__ __forceinline__ uint32_t
 lds_hash(uint64_t k)
 {
@@ -3934,9 +4061,9 @@ lds_hash(uint64_t k)
 
 /* returns the LDS slot of packed key pk, inserting it; -1 if the probe fails */
 __device__ __forceinline__ int
-lds_probe(LdsTable &T, uint64_t pk)
+lds_probe(cplan *P, LdsTable &T, uint64_t pk, const kern_data_store *kds)
 {
-    uint32_t h = (uint32_t)(((uint64_t)lds_hash(pk) * T.n) >> 32);
+    uint32_t h = (uint32_t)(((uint64_t)lds_hash(gb_key_part(P, pk)) * T.n) >> 32);
     for (int i = 0; i < 8; i++)
     {
         unsigned long long cur = T.keys[h];
@@ -3947,7 +4074,11 @@ lds_probe(LdsTable &T, uint64_t pk)
             unsigned long long old = atomicCAS(&T.keys[h], XLDS_EMPTY_KEY, (unsigned long long)pk);
             if (old == XLDS_EMPTY_KEY || old == pk)
                 return (int)h;
+            cur = old;
         }
+        if (P->lds_text && (cur >> 32) == (pk >> 32) &&
+            gb_rows_match(P, kds, (uint32_t)cur, (uint32_t)pk))
+            return (int)h;
         if (++h == T.n)
             h = 0;
     }
@@ -4071,8 +4202,8 @@ lds_init(cplan *P, LdsTable &T)
  * each per group. */
 template <int NR>
 __device__ __forceinline__ void
-lds_flush(cplan *P, LdsTable &T, kern_data_store *kds_final, xpu_task_ctl *ctl,
-          kern_data_store *kds_ovf = nullptr)
+lds_flush(cplan *P, LdsTable &T, const kern_data_store *kds_src, kern_data_store *kds_final,
+          xpu_task_ctl *ctl, kern_data_store *kds_ovf = nullptr)
 {
     int64_t Rfile[NR];
     Lane L;
@@ -4129,7 +4260,7 @@ lds_flush(cplan *P, LdsTable &T, kern_data_store *kds_final, xpu_task_ctl *ctl,
             uint32_t hash = 0;
             if (pending)
             {
-                gb_unpack_key(P, L, T.keys[slot]);
+                gb_unpack_key(P, L, T.keys[slot], kds_src);
                 hash = gb_hash_regs(P, L);
             }
             gb_global(P, L, kds_final, hash, pending, &T, pending ? (int)slot : -1, ctl, kds_ovf);
@@ -4184,7 +4315,7 @@ lds_dump(cplan *P, LdsTable &T, const xpu_kparams &kp)
     {
         unsigned long long key = T.keys[h];
         if (key != XLDS_EMPTY_KEY && T.rows[h] != 0)
-            atomicAdd(&s_cnt[dump_partition(key, np)], 1U);
+            atomicAdd(&s_cnt[dump_partition(gb_key_part(P, key), np)], 1U);
     }
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < np; i += blockDim.x)
@@ -4215,7 +4346,7 @@ lds_dump(cplan *P, LdsTable &T, const xpu_kparams &kp)
             unsigned long long key = T.keys[h];
             if (key != XLDS_EMPTY_KEY && T.rows[h] != 0)
             {
-                const uint32_t part = dump_partition(key, np);
+                const uint32_t part = dump_partition(gb_key_part(P, key), np);
                 const uint64_t idx = s_base[part] + atomicAdd(&s_cnt[part], 1U);
                 if (idx < kp.dump_cap)
                 {
@@ -4230,7 +4361,7 @@ lds_dump(cplan *P, LdsTable &T, const xpu_kparams &kp)
                 }
                 else
                 {
-                    gb_unpack_key(P, L, key);
+                    gb_unpack_key(P, L, key, kp.kds_src);
                     hash = gb_hash_regs(P, L);
                     pending = true;
                     ndirect++;
@@ -4328,7 +4459,7 @@ dump_merge_part(cplan *P, const xpu_kparams &kp, LdsTable &T, uint32_t part)
                 if (i < c1 && ((left >> k) & 1))
                 {
                     const uint64_t *rec = recs + i * rw;
-                    const int slot = lds_probe(T, rec[0]);
+                    const int slot = lds_probe(P, T, rec[0], kp.kds_src);
                     if (slot >= 0)
                         lds_merge_entry(P, T, slot, rec);
                     else
@@ -4337,7 +4468,7 @@ dump_merge_part(cplan *P, const xpu_kparams &kp, LdsTable &T, uint32_t part)
             }
             if (!__syncthreads_or(again != 0))
                 break;
-            lds_flush<NR>(P, T, kp.kds_out, kp.ctl, kp.kds_ovf);
+            lds_flush<NR>(P, T, kp.kds_src, kp.kds_out, kp.ctl, kp.kds_ovf);
             __syncthreads();
             lds_init(P, T);
             __syncthreads();
@@ -4345,7 +4476,7 @@ dump_merge_part(cplan *P, const xpu_kparams &kp, LdsTable &T, uint32_t part)
         }
     }
     __syncthreads();
-    lds_flush<NR>(P, T, kp.kds_out, kp.ctl, kp.kds_ovf);
+    lds_flush<NR>(P, T, kp.kds_src, kp.kds_out, kp.ctl, kp.kds_ovf);
     __syncthreads();
 }
 
@@ -4868,7 +4999,7 @@ pipeline_body(cplan *P, const xpu_kparams &kp)
                     bool direct = true;
                     if (T.n > 0 && gb_row_fast(P, L))
                     {
-                        int slot = lds_probe(T, gb_pack_key(P, L));
+                        int slot = lds_probe(P, T, gb_pack_key(P, L, 0), kds);
                         if (slot >= 0)
                         {
                             lds_update(P, L, T, slot);
@@ -5151,7 +5282,7 @@ pipeline_body(cplan *P, const xpu_kparams &kp)
     if (PREAGG && T.n > 0)
     {
         __syncthreads();
-        lds_flush<NR>(P, T, kp.kds_out, ctl, kp.kds_ovf);
+        lds_flush<NR>(P, T, kp.kds_src, kp.kds_out, ctl, kp.kds_ovf);
     }
     if (cnt_in)
         atomicAdd(&ctl->nitems_in, cnt_in);
@@ -5465,7 +5596,7 @@ join_probe_body(cplan *P, const xpu_kparams &kp)
                     bool direct = true;
                     if (T.n > 0 && gb_row_fast(P, L))
                     {
-                        int slot = lds_probe(T, gb_pack_key(P, L));
+                        int slot = lds_probe(P, T, gb_pack_key(P, L, 0), kds);
                         if (slot >= 0)
                         {
                             lds_update(P, L, T, slot);
@@ -5520,7 +5651,7 @@ join_probe_body(cplan *P, const xpu_kparams &kp)
     if (T.n > 0)
     {
         __syncthreads();
-        lds_flush<NR>(P, T, kp.kds_out, ctl, kp.kds_ovf);
+        lds_flush<NR>(P, T, kp.kds_src, kp.kds_out, ctl, kp.kds_ovf);
     }
     if (cnt_out)
         atomicAdd(&ctl->nitems_out, cnt_out);
@@ -5895,8 +6026,8 @@ scan_agg_range(cplan *P, const xpu_kparams &kp, LdsTable &T, uint64_t wt_first,
             uint64_t pk = 0;
             if (ok && T.n > 0 && gb_row_fast(P, L))
             {
-                pk = gb_pack_key(P, L);
-                int slot = lds_probe(T, pk);
+                pk = gb_pack_key(P, L, (uint32_t)row);
+                int slot = lds_probe(P, T, pk, kds);
                 if (slot >= 0)
                 {
                     lds_update(P, L, T, slot);
@@ -6007,7 +6138,7 @@ scan_agg_body(cplan *P, const xpu_kparams &kp)
         if (kp.dump)
             lds_dump<NR>(P, T, kp);
         else
-            lds_flush<NR>(P, T, kp.kds_out, kp.ctl, kp.kds_ovf);
+            lds_flush<NR>(P, T, kp.kds_src, kp.kds_out, kp.ctl, kp.kds_ovf);
     }
     scan_agg_report(kp.ctl, W);
 }
@@ -6045,14 +6176,14 @@ spill_fold_range(cplan *P, const xpu_kparams &kp, LdsTable &T, uint64_t lo, uint
         bool fail = false;
         if (pk != XLDS_EMPTY_KEY)
         {
-            gb_unpack_key(P, L, pk);
+            gb_unpack_key(P, L, pk, kp.kds_src);
             for (int j = 0; j < (int)P->spill_nregs; j++)
             {
                 const int r = P->spill_regs[j];
                 L.R[r] = (int64_t)kp.spill[i * rec_words + 1 + j];
                 SETNULL(L, r, 0);
             }
-            int slot = lds_probe(T, pk);
+            int slot = lds_probe(P, T, pk, kp.kds_src);
             if (slot >= 0)
                 lds_update(P, L, T, slot);
             else
@@ -6066,7 +6197,7 @@ spill_fold_range(cplan *P, const xpu_kparams &kp, LdsTable &T, uint64_t lo, uint
             __syncthreads();
             if (fail)
             {
-                int slot = lds_probe(T, pk);
+                int slot = lds_probe(P, T, pk, kp.kds_src);
                 if (slot >= 0)
                 {
                     lds_update(P, L, T, slot);
@@ -6150,7 +6281,7 @@ batch_leave(cplan *P, const xpu_kparams &kp, LdsTable &T, const xbatch_frag &f)
         lds_dump<NR>(P, T, k);
     }
     else
-        lds_flush<NR>(P, T, f.kds_final, f.ctl);
+        lds_flush<NR>(P, T, f.kds_src, f.kds_final, f.ctl);
 }
 
 template <int NR, int RPT, class PROG>

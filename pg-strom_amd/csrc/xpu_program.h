@@ -273,7 +273,10 @@ typedef struct
     uint8_t     spill_ok;
     uint8_t     spill_nregs;
     uint8_t     spill_regs[XP_MAX_SPILL];
-    uint8_t     __pad3[6];
+    uint8_t     lds_text;           /* lds_fast with text keys: entries name their group
+                                       by hash and a row of the chunk */
+    uint8_t     __pad3[5];
+    uint16_t    key_ld[XP_MAX_KEYS];    /* lds_text: the column load of each key (op) */
     xattr       keys[XP_MAX_KEYS];
     uint8_t     key_bits[XP_MAX_KEYS];  /* packed width of each key in bits */
     xagg        aggs[XP_MAX_PROJ];

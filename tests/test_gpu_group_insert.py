@@ -98,3 +98,27 @@ def test_batch_of_uneven_fragments(gpu, jit, graph):
         assert_groups_equal(s.final(), exp, acts)
         s.close()
     dev.free()
+
+
+@pytest.mark.parametrize("lds_nents", [96, 1500])
+def test_text_groups_beyond_a_table(gpu, jit, lds_nents):
+    """Text keys name their group by a row of the chunk through spill records
+    and dumps: 20,000 texts that share prefixes, some of one byte, and an int4
+    key beside them, over heap pages and an Arrow chunk."""
+    r = np.random.default_rng(lds_nents)
+    n = 60_000
+    pick = r.integers(0, 20_000, size=n)
+    cols = [kds.Column("key", "text", [b"prefix-of-many-%d" % i if i > 200 else b"%c" % (32 + i % 90)
+                                       for i in pick], r.random(n) < 0.01),
+            kds.Column("k2", "int4", (pick % 3).astype(np.int32), r.random(n) < 0.01)] + _args(n, r)
+    plan = cg.Plan([(c.name, c.typname) for c in cols])
+    kv = [plan.scan_var("key"), plan.scan_var("k2")]
+    tlist = W.preagg_tlist(plan, kv[0], *[plan.scan_var(k) for k in ("v", "w", "x")])
+    tlist.append((abi.KAGG_ACTION__VREF, kv[1], ("k2", "int4")))
+    plan.set_groupby(tlist)
+    blob = plan.build(final_nrows=20_000)
+    src = kds.build_arrow_kds(cols)
+    exp = run_oracle_groupby(blob, [src])
+    for chunk in (src, kds.build_block_kds(cols)):
+        fin = run_gpu_groupby(blob, [chunk], tuning=dict(jit=jit, lds_nents=lds_nents))
+        assert_groups_equal(fin, exp, [a for a, _, _ in tlist])
