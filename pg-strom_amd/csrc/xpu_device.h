@@ -6248,24 +6248,38 @@ spill_agg_body(cplan *P, const xpu_kparams &kp)
  * 91M rows, 11.3 + 2.4 ms of a 13.8 ms batch.)
  * ------------------------------------------------------------------ */
 
+/* fragments and work items are read through the constant address space at
+ * wave-uniform numbers (a number taken from LDS is not uniform to the
+ * compiler: with it, every column address and bound of a fragment lived in
+ * vector registers and the scan pass of 24 fragments, 91M rows, took 8.2 ms) */
+typedef const XCONST xbatch_frag cbatch_frag;
+typedef const XCONST xbatch_item cbatch_item;
+typedef const XCONST xbatch_sitem cbatch_sitem;
+
+__device__ __forceinline__ cbatch_frag *
+batch_frag(const xpu_kparams &kp, uint32_t f)
+{
+    return (cbatch_frag *)(uintptr_t)kp.batch_frags + f;
+}
+
 /* the task parameters of fragment f on top of the launch's common ones */
 __device__ __forceinline__ xpu_kparams
-batch_kparams(const xpu_kparams &kp, const xbatch_frag &f)
+batch_kparams(const xpu_kparams &kp, cbatch_frag *f)
 {
     xpu_kparams k = kp;
-    k.kds_src = f.kds_src;
-    k.kds_out = f.kds_final;
-    k.ctl = f.ctl;
-    k.const_pool = f.const_pool;
-    k.params = f.params;
-    k.param_nulls = f.param_nulls;
-    k.spill = f.spill;
-    k.spill_cap = f.spill_cap;
-    k.dump = f.dump;
-    k.dump_cap = f.dump_cap;
-    k.dump_next = f.dump_next;
+    k.kds_src = f->kds_src;
+    k.kds_out = f->kds_final;
+    k.ctl = f->ctl;
+    k.const_pool = f->const_pool;
+    k.params = f->params;
+    k.param_nulls = f->param_nulls;
+    k.spill = f->spill;
+    k.spill_cap = f->spill_cap;
+    k.dump = f->dump;
+    k.dump_cap = f->dump_cap;
+    k.dump_next = f->dump_next;
     k.row_begin = 0;
-    k.row_end = f.nrows;
+    k.row_end = f->nrows;
     return k;
 }
 
@@ -6273,7 +6287,7 @@ batch_kparams(const xpu_kparams &kp, const xbatch_frag &f)
  * its kds_final where the plan has no spill records (and so no dumps) */
 template <int NR>
 __device__ __forceinline__ void
-batch_leave(cplan *P, const xpu_kparams &kp, LdsTable &T, const xbatch_frag &f)
+batch_leave(cplan *P, const xpu_kparams &kp, LdsTable &T, cbatch_frag *f)
 {
     if (kp.dump_nparts > 0)
     {
@@ -6281,7 +6295,7 @@ batch_leave(cplan *P, const xpu_kparams &kp, LdsTable &T, const xbatch_frag &f)
         lds_dump<NR>(P, T, k);
     }
     else
-        lds_flush<NR>(P, T, f.kds_src, f.kds_final, f.ctl);
+        lds_flush<NR>(P, T, f->kds_src, f->kds_final, f->ctl);
 }
 
 template <int NR, int RPT, class PROG>
@@ -6302,39 +6316,39 @@ batch_agg_body(cplan *P, const xpu_kparams &kp)
         if (threadIdx.x == 0)
             s_item = atomicAdd(kp.batch_ticket, 1U);
         __syncthreads();
-        const uint32_t it = s_item;
+        const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
         __syncthreads();
         if (it >= kp.batch_nitems)
             break;
-        const xbatch_item item = kp.batch_items[it];
-        if ((int)item.frag != cur)
+        cbatch_item *item = (cbatch_item *)(uintptr_t)kp.batch_items + it;
+        if ((int)item->frag != cur)
         {
             if (cur >= 0)
             {
-                const xbatch_frag &fc = kp.batch_frags[cur];
+                cbatch_frag *fc = batch_frag(kp, (uint32_t)cur);
                 if (T.n > 0)
                 {
                     batch_leave<NR>(P, kp, T, fc);
                     __syncthreads();
                     lds_init(P, T);
                 }
-                scan_agg_report(fc.ctl, W);
+                scan_agg_report(fc->ctl, W);
             }
             __syncthreads();
-            cur = (int)item.frag;
+            cur = (int)item->frag;
         }
-        xpu_kparams k = batch_kparams(kp, kp.batch_frags[item.frag]);
-        k.row_begin = item.row_begin;
-        k.row_end = item.row_end;
+        xpu_kparams k = batch_kparams(kp, batch_frag(kp, item->frag));
+        k.row_begin = item->row_begin;
+        k.row_end = item->row_end;
         scan_agg_range<NR, RPT, PROG>(P, k, T, wid, nwaves, W);
         __syncthreads();
     }
     if (cur >= 0)
     {
-        const xbatch_frag &fc = kp.batch_frags[cur];
+        cbatch_frag *fc = batch_frag(kp, (uint32_t)cur);
         if (T.n > 0)
             batch_leave<NR>(P, kp, T, fc);
-        scan_agg_report(fc.ctl, W);
+        scan_agg_report(fc->ctl, W);
     }
 }
 
@@ -6395,15 +6409,16 @@ batch_spill_body(cplan *P, const xpu_kparams &kp)
         if (threadIdx.x == 0)
             s_item = atomicAdd(&kp.batch_ticket[1], 1U);
         __syncthreads();
-        const uint32_t it = s_item;
+        const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
         __syncthreads();
         if (it >= nsitems)
             break;
-        const xbatch_sitem si = kp.batch_sitems[it];
-        const xpu_kparams k = batch_kparams(kp, kp.batch_frags[si.frag]);
+        /* (written by the setup kernel before this one) */
+        cbatch_sitem *si = (cbatch_sitem *)(uintptr_t)kp.batch_sitems + it;
+        const xpu_kparams k = batch_kparams(kp, batch_frag(kp, si->frag));
         lds_init(P, T);
         __syncthreads();
-        spill_fold_range<NR>(P, k, T, si.lo, si.hi);
+        spill_fold_range<NR>(P, k, T, si->lo, si->hi);
         __syncthreads();
         lds_dump<NR>(P, T, k);
         __syncthreads();
@@ -6422,7 +6437,7 @@ batch_merge_body(cplan *P, const xpu_kparams &kp)
     const uint32_t n = kp.batch_nfrags * kp.dump_nparts;
     for (uint32_t it = blockIdx.x; it < n; it += gridDim.x)
     {
-        const xpu_kparams k = batch_kparams(kp, kp.batch_frags[it / kp.dump_nparts]);
+        const xpu_kparams k = batch_kparams(kp, batch_frag(kp, it / kp.dump_nparts));
         dump_merge_part<NR>(P, k, T, it % kp.dump_nparts);
     }
 }
