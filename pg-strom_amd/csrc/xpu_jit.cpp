@@ -92,7 +92,7 @@ xpu_jit_source(const xplan *P, int kind, int param)
 
     std::string s;
     s.reserve(8 * nbytes + 4096);
-    s += "#include \"xpu_device.h\"\n\n";
+    s += "#define XPU_PLAN_CONST 1\n#include \"xpu_device.h\"\n\n";
     append(s, "__constant__ const unsigned char xjit_plan[%zu] __attribute__((aligned(16))) = {", nbytes);
     for (size_t i = 0; i < nbytes; i++)
         append(s, "%s%u", i == 0 ? "\n    " : (i % 32 == 0 ? ",\n    " : ","), b[i]);
