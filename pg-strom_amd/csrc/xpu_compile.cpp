@@ -1847,6 +1847,14 @@ xpu_compile_session(const kern_session_info *s, size_t length, xpu_compiled *out
             }
             P->spill_ok = fits ? 1 : 0;
             P->spill_nregs = fits ? (uint8_t)n : 0;
+            for (int j = 0; j < nattrs; j++)
+            {
+                xagg *ag = &P->aggs[j];
+                ag->nul = 0xff;
+                for (int k = 0; k < P->spill_nregs; k++)
+                    if (ag->action != KAGG_ACTION__VREF && ag->arg_reg == P->spill_regs[k])
+                        ag->nul = (uint8_t)k;
+            }
         }
         P->lds_n64 = lds_n64;
         P->lds_n32 = lds_n32;

@@ -211,6 +211,8 @@ typedef struct
     int8_t      lds64;      /* 8-byte LDS field array of this action (-1: none) */
     int8_t      lds32;      /* 4-byte LDS field array of this action (-1: none) */
     uint16_t    num_scale;  /* PSUM/PAVG_NUMERIC: decimal scale of the sum */
+    uint8_t     nul;        /* its argument among spill_regs (0xff: none) */
+    uint8_t     __pad[3];
 } xagg;
 
 /* a depth-0 fixed-width column loaded by the scan kernel's tile prologue */

@@ -496,6 +496,20 @@ lds_bytes_for(const xplan *P, uint32_t nents)
     return (size_t)nents * P->lds_entry_bytes;
 }
 
+/* bytes of a spill record and words of a dump record, with their NULL parts
+ * (a chunk without validity bitmaps has shorter ones) */
+uint64_t
+spill_rec_bytes(const xplan *P)
+{
+    return 8ULL * (2 + P->spill_nregs);
+}
+
+uint64_t
+dump_rec_words(const xplan *P)
+{
+    return 1 + P->lds_n64 + (1 + P->lds_n32 + P->spill_nregs + 1) / 2;
+}
+
 /* plans without joins run the scan + group-by kernel */
 bool
 uses_scan_agg(const xpuhip_session *s)
@@ -1642,7 +1656,7 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
      * the rows above; rows beyond it merge into kds_final directly */
     if (spill)
     {
-        uint64_t rec = 8ULL * (1 + P->spill_nregs);
+        uint64_t rec = spill_rec_bytes(P);
         const uint64_t all = nrows + (uint64_t)grid * (block / 64) * XSPILL_CHUNK;
         /* a table of a few entries folds next to nothing before it dumps */
         const uint64_t room = lds_nents >= 1024 ? XPU_SPILL_BYTES / rec : 1ULL << 20;
@@ -1655,7 +1669,7 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
          * partial-state records; one block per partition merges each group
          * into kds_final once */
         uint32_t nparts = (uint32_t)g_dev.ncu < XP_DUMP_MAXPARTS ? (uint32_t)g_dev.ncu : XP_DUMP_MAXPARTS;
-        uint64_t rw = 1 + P->lds_n64 + (1 + P->lds_n32 + 1) / 2;
+        uint64_t rw = dump_rec_words(P);
         /* one table per block from the scan pass plus the spill pass's
          * dumps of full tables: a record for every spilled row at most, and
          * beyond XPU_DUMP_BYTES room for eight tables per block; an eighth
@@ -2380,8 +2394,8 @@ xpuhip_task_exec_device_noalloc(xpuhip_session *s, const kern_data_store *d_src,
     {
         const uint32_t nparts = (uint32_t)g_dev.ncu < XP_DUMP_MAXPARTS ? (uint32_t)g_dev.ncu
                                                                       : XP_DUMP_MAXPARTS;
-        const uint64_t rw = 1 + P->lds_n64 + (1 + P->lds_n32 + 1) / 2;
-        const uint64_t rec = 8ULL * (1 + P->spill_nregs);
+        const uint64_t rw = dump_rec_words(P);
+        const uint64_t rec = spill_rec_bytes(P);
         const size_t next_bytes = (8ULL * XP_DUMP_MAXPARTS + 255) & ~(size_t)255;
         const size_t rest = avail - next_bytes;
         const uint64_t dump_cap = (rest / 2) / (nparts * rw * 8);
@@ -3165,7 +3179,7 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     /* spill regions: an eighth of each fragment's rows (at least 64K records),
      * scaled down to the batch's spill budget */
     const bool spill = P->spill_ok && lds_nents > 0;
-    const uint64_t rec = 8ULL * (1 + P->spill_nregs);
+    const uint64_t rec = spill_rec_bytes(P);
     std::vector<uint64_t> caps(ntasks, 0);
     uint64_t spill_recs = 0;
     if (spill)
@@ -3194,7 +3208,7 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
      * its spilled rows, an eighth more for uneven partitions; entries past a
      * partition's capacity merge into kds_final directly */
     uint32_t nparts = 0;
-    const uint64_t rw = 1 + P->lds_n64 + (1 + P->lds_n32 + 1) / 2;
+    const uint64_t rw = dump_rec_words(P);
     std::vector<uint64_t> dcaps(ntasks, 0);
     uint64_t dump_recs = 0;
     if (spill)

@@ -122,3 +122,63 @@ def test_text_groups_beyond_a_table(gpu, jit, lds_nents):
     for chunk in (src, kds.build_block_kds(cols)):
         fin = run_gpu_groupby(blob, [chunk], tuning=dict(jit=jit, lds_nents=lds_nents))
         assert_groups_equal(fin, exp, [a for a, _, _ in tlist])
+
+
+@pytest.mark.parametrize("lds_nents", [64, 1200])
+@pytest.mark.parametrize("null_frac", [0.05, 0.9])
+def test_null_arguments_through_the_tables(gpu, jit, lds_nents, null_frac):
+    """Arguments with validity bitmaps: NULLs are counted per entry in the
+    tables, spill records and dumps (every action that skips a NULL), and one
+    column of the chunk is NULL throughout."""
+    r = np.random.default_rng(int(100 * null_frac) + lds_nents)
+    n = 40_000
+    a = _args(n, r)
+    for c in a[:2]:
+        c.nulls = r.random(n) < null_frac
+    a[2].nulls = np.ones(n, dtype=bool)
+    cols = [kds.Column("key", "int4", r.integers(0, 3000, size=n).astype(np.int32),
+                       r.random(n) < 0.05)] + a
+    plan = cg.Plan([(c.name, c.typname) for c in cols])
+    key, v, w, x = (plan.scan_var(k) for k in ("key", "v", "w", "x"))
+    tlist = [(abi.KAGG_ACTION__NROWS_ANY, None, ("n", "int8")),
+             (abi.KAGG_ACTION__NROWS_COND, v, ("nv", "int8")),
+             (abi.KAGG_ACTION__PSUM_INT64, v, ("sv", "bytea")),
+             (abi.KAGG_ACTION__PMIN_INT64, v, ("mv", "bytea")),
+             (abi.KAGG_ACTION__STDDEV, w, ("dw", "bytea")),
+             (abi.KAGG_ACTION__PMAX_FP64, w, ("xw", "bytea")),
+             (abi.KAGG_ACTION__PSUM_INT, x, ("sx", "bytea")),
+             (abi.KAGG_ACTION__PMAX_INT32, x, ("xx", "bytea")),
+             (abi.KAGG_ACTION__VREF, key, ("key", "int4"))]
+    plan.set_groupby(tlist)
+    blob = plan.build(final_nrows=3000)
+    src = kds.build_arrow_kds(cols)
+    fin = run_gpu_groupby(blob, [src], tuning=dict(jit=jit, lds_nents=lds_nents))
+    # sums of squares of uniform [0, 1) values: addends of one sign
+    assert_groups_equal(fin, run_oracle_groupby(blob, [src]), [t[0] for t in tlist])
+
+
+def test_batch_of_text_keys(gpu, jit):
+    """Fragments grouped by a text column in one launch: entries name rows of
+    their own fragment's window."""
+    r = np.random.default_rng(4)
+    n = 30_000
+    cols = [kds.Column("key", "text", [b"k%d" % i for i in r.integers(0, 4000, size=n)],
+                       r.random(n) < 0.02)] + _args(n, r)
+    cols[2].nulls = r.random(n) < 0.1
+    blob = W.preagg_query(cols)
+    acts = [a for a, _, _ in W.preagg_tlist(None, cols[0], None, None, None)]
+    wins = [(0, 30_000), (64, 1), (8_000, 9_999)]
+    chunk = kds.build_arrow_kds(cols)
+    hdrs = kds.window_headers(chunk, wins, len(wins) * 1024, 1024)
+    dev = xpuhip.DeviceBuffer(len(hdrs) + len(chunk), np.concatenate([hdrs, chunk]))
+    sess = [xpuhip.Session(blob) for _ in wins]
+    for s in sess:
+        s.set_tuning(jit=jit, lds_nents=1024)
+    xpuhip.batch_exec([(s, dev.ptr + i * 1024, w[1]) for i, (s, w) in enumerate(zip(sess, wins))],
+                      graph=False)
+    for s, (r0, m) in zip(sess, wins):
+        keep = (np.arange(n) >= r0) & (np.arange(n) < r0 + m)
+        part = kds.build_arrow_kds(datagen.take_rows(cols, keep))
+        assert_groups_equal(s.final(), run_oracle_groupby(blob, [part]), acts)
+        s.close()
+    dev.free()
