@@ -330,7 +330,7 @@ typedef struct
 int xpu_launch_sort_keys(const xsort_params *sp, void *stream);
 int xpu_launch_sort_pass(const uint64_t *words_in, const uint32_t *idx_in, uint64_t *words_out,
                          uint32_t *idx_out, uint32_t n, uint32_t nwords, uint32_t word,
-                         uint64_t base, uint32_t shift, uint32_t *counts,
+                         uint64_t base, uint32_t shift, uint32_t carry, uint32_t *counts,
                          void *stream);          /* counts: 256 * (ntiles + 1) */
 int xpu_launch_sort_permute(const uint64_t *rowindex, const uint32_t *idx, uint64_t *out,
                             uint32_t n, void *stream);

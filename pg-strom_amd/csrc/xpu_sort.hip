@@ -80,20 +80,12 @@ sort_enc_f64(uint64_t b)
     return (b & 0x8000000000000000ULL) ? ~b : (b | 0x8000000000000000ULL);
 }
 
-__global__ void __launch_bounds__(XSORT_BLOCK)
-xpu_sort_keys_kernel(xsort_params sp)
+/* the key words of item i, whose tuple is t (in LDS or in the final buffer),
+ * and the block's least and greatest value of each word */
+__device__ __forceinline__ void
+sort_item_keys(const xsort_params &sp, const kern_tupitem *t, uint32_t i, bool valid,
+               unsigned long long *s_min, unsigned long long *s_max)
 {
-    __shared__ unsigned long long s_min[XSORT_MAX_WORDS];
-    __shared__ unsigned long long s_max[XSORT_MAX_WORDS];
-    const uint32_t nw = sp.nwords;
-    if (threadIdx.x < nw)
-    {
-        s_min[threadIdx.x] = ~0ULL;
-        s_max[threadIdx.x] = 0;
-    }
-    __syncthreads();
-    const uint32_t i = blockIdx.x * XSORT_BLOCK + threadIdx.x;
-    const bool valid = i < sp.n;
     /* one walk of the tuple finds every key attribute (the attribute walk
      * of kern_fetch_minimal_tuple_attr: NULL bitmap, alignment of fixed
      * values and of 4-byte varlena headers, 1- and 4-byte header lengths) */
@@ -103,8 +95,6 @@ xpu_sort_keys_kernel(xsort_params sp)
         kptr[k] = nullptr;
     if (valid)
     {
-        const kern_tupitem *t = (const kern_tupitem *)
-            ((const char *)sp.kds + sp.kds->length - sp.rowindex[i]);
         const int natts = t->t_infomask2 & HEAP_NATTS_MASK;
         const int last = (int)sp.max_anum < natts ? (int)sp.max_anum : natts;
         const bool hasnull = (t->t_infomask & HEAP_HASNULL) != 0;
@@ -292,6 +282,49 @@ xpu_sort_keys_kernel(xsort_params sp)
             }
         }
     }
+}
+
+__global__ void __launch_bounds__(XSORT_BLOCK)
+xpu_sort_keys_kernel(xsort_params sp)
+{
+    __shared__ unsigned long long s_min[XSORT_MAX_WORDS];
+    __shared__ unsigned long long s_max[XSORT_MAX_WORDS];
+    const uint32_t nw = sp.nwords;
+    if (threadIdx.x < nw)
+    {
+        s_min[threadIdx.x] = ~0ULL;
+        s_max[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    const uint32_t i = blockIdx.x * XSORT_BLOCK + threadIdx.x;
+    const bool valid = i < sp.n;
+    /* The first 128 bytes of each tuple (a group tuple of up to five or six
+     * aggregates) go to LDS with coalesced loads, and the walk reads them
+     * there: walked in memory, each of its loads touches a line per lane
+     * (950,000 items: 0.33 ms that way, 0.09 ms this way).  136 bytes apart, so that the lanes
+     * spread over the banks. */
+    __shared__ __attribute__((aligned(8))) char s_tup[XSORT_BLOCK / 64][64 * 136];
+    const uint32_t lane = __lane_id();
+    char *mine = s_tup[threadIdx.x / 64];
+    const char *kds_end = (const char *)sp.kds + sp.kds->length;
+    const kern_tupitem *t = valid ? (const kern_tupitem *)(kds_end - sp.rowindex[i]) : nullptr;
+    for (uint32_t r = 0; r < 16; r++)
+    {
+        const uint32_t src = 4 * r + (lane >> 4);
+        const char *a = (const char *)__shfl((unsigned long long)(uintptr_t)t, (int)src);
+        const char *w = a + 8 * (lane & 15);
+        if (a && w + 8 <= kds_end)
+            *(uint64_t *)(mine + 136 * src + 8 * (lane & 15)) = *(const uint64_t *)w;
+    }
+    /* (a wave reads what it staged itself) */
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const kern_tupitem *st = (const kern_tupitem *)(mine + 136 * lane);
+    if (__ballot(valid && st->t_len > 128) == 0)
+        sort_item_keys(sp, st, i, valid, s_min, s_max);
+    else
+        sort_item_keys(sp, t, i, valid, s_min, s_max);
     if (valid)
         sp.idx[i] = i;
     __syncthreads();
@@ -380,7 +413,7 @@ xpu_sort_scan_kernel(uint32_t *counts, uint32_t ntiles, uint32_t *totals)
 __global__ void __launch_bounds__(XSORT_BLOCK)
 xpu_sort_scatter_kernel(const uint64_t *words_in, const uint32_t *idx_in, uint64_t *words_out,
                         uint32_t *idx_out, uint32_t n, uint32_t nwords, uint32_t word,
-                        uint64_t wbase, uint32_t shift, const uint32_t *counts,
+                        uint64_t wbase, uint32_t shift, uint32_t carry, const uint32_t *counts,
                         const uint32_t *totals)
 {
     __shared__ uint32_t run[256];
@@ -420,7 +453,8 @@ xpu_sort_scatter_kernel(const uint64_t *words_in, const uint32_t *idx_in, uint64
             for (uint32_t w2 = 0; w2 < wave; w2++)
                 pos += wc[w2][d];
             for (uint32_t k = 0; k < nwords; k++)
-                words_out[(uint64_t)k * n + pos] = words_in[(uint64_t)k * n + j];
+                if ((carry >> k) & 1U)
+                    words_out[(uint64_t)k * n + pos] = words_in[(uint64_t)k * n + j];
             idx_out[pos] = idx_in[j];
         }
         __syncthreads();
@@ -709,11 +743,12 @@ xpu_launch_sort_keys(const xsort_params *sp, void *stream)
 }
 
 /* one stable pass by the digit ((words[word] - base) >> shift) & 0xff;
- * counts holds 256 * (ceil(n / XSORT_TILE) + 1) entries */
+ * carry: the words that later passes read (bit k: word k), the others are
+ * left behind; counts holds 256 * (ceil(n / XSORT_TILE) + 1) entries */
 extern "C" int
 xpu_launch_sort_pass(const uint64_t *words_in, const uint32_t *idx_in, uint64_t *words_out,
                      uint32_t *idx_out, uint32_t n, uint32_t nwords, uint32_t word,
-                     uint64_t base, uint32_t shift, uint32_t *counts, void *stream)
+                     uint64_t base, uint32_t shift, uint32_t carry, uint32_t *counts, void *stream)
 {
     if (n == 0)
         return 0;
@@ -725,7 +760,8 @@ xpu_launch_sort_pass(const uint64_t *words_in, const uint32_t *idx_in, uint64_t 
                        counts, ntiles, totals);
     hipLaunchKernelGGL(xpu_sort_scatter_kernel, dim3(ntiles), dim3(XSORT_BLOCK), 0,
                        (hipStream_t)stream, words_in, idx_in, words_out, idx_out, n, nwords,
-                       word, base, shift, (const uint32_t *)counts, (const uint32_t *)totals);
+                       word, base, shift, carry, (const uint32_t *)counts,
+                       (const uint32_t *)totals);
     return (int)hipGetLastError();
 }
 
