@@ -40,7 +40,8 @@ typedef struct
     uint32_t    join_passes;        /* XPUHIP_JOIN_PASSES_*: group-by joins in passes */
 } xpuhip_tuning;
 
-#define XPUHIP_JIT_AUTO     0       /* specialize chunks of >= 1,000,000 rows */
+#define XPUHIP_JIT_AUTO     0       /* specialize chunks of >= 1,000,000 rows, and
+                                       any chunk of a plan that has run as many */
 #define XPUHIP_JIT_ON       1       /* always specialize */
 #define XPUHIP_JIT_OFF      2       /* always run the op interpreter */
 

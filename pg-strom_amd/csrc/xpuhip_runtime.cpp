@@ -140,7 +140,7 @@ ensure_device(kern_errorbuf *eb)
  * that size wait until the driver has cleared the freed memory (a 2M-row
  * star query opened and closed in a row: 42 ms a query, 1.9 ms with the
  * buffers kept).  Buffers are reused
- * by rounded size; at most DEVPOOL_KEEP_BYTES stay idle, all go back when an
+ * by device and rounded size; at most DEVPOOL_KEEP_BYTES stay idle, all go back when an
  * allocation fails or at xpuhip_shutdown.  A buffer is given back only after
  * the work that used it has completed (every entry point waits for its own). */
 #define DEVPOOL_KEEP_BYTES      (8ULL << 30)
@@ -149,8 +149,9 @@ ensure_device(kern_errorbuf *eb)
 struct DevPool
 {
     std::mutex  lock;
-    std::map<void *, size_t> live;                  /* buffer -> rounded size */
-    std::multimap<size_t, void *> idle;
+    typedef std::pair<int, size_t> Key;             /* device, rounded size */
+    std::map<void *, Key> live;
+    std::multimap<Key, void *> idle;
     size_t      idle_bytes = 0;
 
     /* at most an eighth more than asked for */
@@ -166,15 +167,16 @@ struct DevPool
     alloc(void **p, size_t n)
     {
         const size_t sz = round_up(n);
+        const Key key(g_dev.id, sz);
         {
             std::lock_guard<std::mutex> g(lock);
-            auto it = idle.find(sz);
+            auto it = idle.find(key);
             if (it != idle.end())
             {
                 *p = it->second;
                 idle.erase(it);
                 idle_bytes -= sz;
-                live[*p] = sz;
+                live[*p] = key;
                 return hipSuccess;
             }
         }
@@ -188,7 +190,7 @@ struct DevPool
         if (rc == hipSuccess)
         {
             std::lock_guard<std::mutex> g(lock);
-            live[*p] = sz;
+            live[*p] = key;
         }
         return rc;
     }
@@ -202,11 +204,12 @@ struct DevPool
             auto it = live.find(p);
             if (it != live.end())
             {
-                const size_t sz = it->second;
+                const Key key = it->second;
+                const size_t sz = key.second;
                 live.erase(it);
                 if (idle_bytes + sz <= DEVPOOL_KEEP_BYTES && idle.size() < DEVPOOL_KEEP_COUNT)
                 {
-                    idle.emplace(sz, p);
+                    idle.emplace(key, p);
                     idle_bytes += sz;
                     return;
                 }
@@ -217,7 +220,7 @@ struct DevPool
     void
     trim()
     {
-        std::multimap<size_t, void *> gone;
+        std::multimap<Key, void *> gone;
         {
             std::lock_guard<std::mutex> g(lock);
             gone.swap(idle);
