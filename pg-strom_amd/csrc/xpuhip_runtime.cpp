@@ -292,18 +292,18 @@ scratch_destroy(Scratch *s)
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     if (s->d_ctl) (void)hipFree(s->d_ctl);
     if (s->h_ctl) (void)hipHostFree(s->h_ctl);
-    if (s->d_status) (void)hipFree(s->d_status);
-    if (s->d_spill) (void)hipFree(s->d_spill);
-    if (s->d_dump) (void)hipFree(s->d_dump);
-    if (s->d_dump_next) (void)hipFree(s->d_dump_next);
-    if (s->d_src) (void)hipFree(s->d_src);
-    if (s->d_dst) (void)hipFree(s->d_dst);
+    if (s->d_status) g_pool.free(s->d_status);
+    if (s->d_spill) g_pool.free(s->d_spill);
+    if (s->d_dump) g_pool.free(s->d_dump);
+    if (s->d_dump_next) g_pool.free(s->d_dump_next);
+    if (s->d_src) g_pool.free(s->d_src);
+    if (s->d_dst) g_pool.free(s->d_dst);
     for (int i = 0; i < 2; i++)
-        if (s->d_rec[i]) (void)hipFree(s->d_rec[i]);
-    if (s->d_rec_cnt) (void)hipFree(s->d_rec_cnt);
-    if (s->d_block_status) (void)hipFree(s->d_block_status);
-    if (s->d_tiles) (void)hipFree(s->d_tiles);
-    if (s->d_hmeta) (void)hipFree(s->d_hmeta);
+        if (s->d_rec[i]) g_pool.free(s->d_rec[i]);
+    if (s->d_rec_cnt) g_pool.free(s->d_rec_cnt);
+    if (s->d_block_status) g_pool.free(s->d_block_status);
+    if (s->d_tiles) g_pool.free(s->d_tiles);
+    if (s->d_hmeta) g_pool.free(s->d_hmeta);
     if (s->h_hstat) (void)hipHostFree(s->h_hstat);
     if (s->h_final) (void)hipHostFree(s->h_final);
     if (s->evh0) (void)hipEventDestroy(s->evh0);
@@ -315,17 +315,22 @@ scratch_destroy(Scratch *s)
     delete s;
 }
 
+/* a scratch buffer of at least need bytes.  Its owner's work has completed,
+ * so a buffer too small goes to the pool: hipFree would wait for every
+ * stream of the process, and powers of two up to 512 MiB make few sizes. */
 bool
 grow(char **p, size_t *cap, size_t need, kern_errorbuf *eb)
 {
     if (*cap >= need)
         return true;
-    if (*p)
-        (void)hipFree(*p);
+    g_pool.free(*p);
     *p = nullptr;
     *cap = 0;
     size_t sz = need + (need >> 3);
-    if (!hip_ok(hipMalloc((void **)p, sz), eb, "hipMalloc"))
+    if (need <= (512ULL << 20))
+        for (sz = 256; sz < need; sz <<= 1)
+            ;
+    if (!hip_ok(g_pool.alloc((void **)p, sz), eb, "hipMalloc"))
         return false;
     *cap = sz;
     return true;
@@ -424,7 +429,7 @@ scratch_trim(Scratch *x)
     auto trim = [](char **p, size_t *cap) {
         if (*p && *cap > XPU_IDLE_KEEP_BYTES)
         {
-            (void)hipFree(*p);
+            g_pool.free(*p);
             *p = nullptr;
             *cap = 0;
         }
@@ -1664,10 +1669,14 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
         /* a table of a few entries folds next to nothing before it dumps */
         const uint64_t room = lds_nents >= 1024 ? XPU_SPILL_BYTES / rec : 1ULL << 20;
         const uint64_t nrec = std::min<uint64_t>(all, std::max<uint64_t>(nrows / 4, room));
-        if (!grow((char **)&x->d_spill, &x->spill_cap, nrec * rec, eb))
+        /* from a million rows on, the same buffer for any of them: a backend's
+         * queries differ in size, and one that grows its scratch waits for
+         * the driver */
+        const bool large = nrows >= (1ULL << 20) && lds_nents >= 1024;
+        if (!grow((char **)&x->d_spill, &x->spill_cap, (large ? std::max(nrec, room) : nrec) * rec, eb))
             return ERRCODE_DEVICE_ERROR;
         kp.spill = x->d_spill;
-        kp.spill_cap = x->spill_cap / rec;
+        kp.spill_cap = std::min<uint64_t>(x->spill_cap / rec, nrec + nrec / 8);
         /* LDS entries leave the scan and spill passes as hash-partitioned
          * partial-state records; one block per partition merges each group
          * into kds_final once */
@@ -1677,9 +1686,9 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
          * dumps of full tables: a record for every spilled row at most, and
          * beyond XPU_DUMP_BYTES room for eight tables per block; an eighth
          * more for uneven partitions */
-        const uint64_t ndump = std::min<uint64_t>((uint64_t)grid * lds_nents + std::min<uint64_t>(nrec, nrows),
-                                                  std::max<uint64_t>(8ULL * grid * lds_nents,
-                                                                     XPU_DUMP_BYTES / (8 * rw)));
+        const uint64_t dmax = std::max<uint64_t>(8ULL * grid * lds_nents, XPU_DUMP_BYTES / (8 * rw));
+        const uint64_t ndump = large ? dmax : std::min<uint64_t>((uint64_t)grid * lds_nents +
+                                                                 std::min<uint64_t>(nrec, nrows), dmax);
         uint64_t per_part = ndump / nparts * 9 / 8 + 1024;
         if (!grow((char **)&x->d_dump, &x->dump_cap, per_part * nparts * rw * 8, eb) ||
             !grow((char **)&x->d_dump_next, &x->dump_next_cap, 8ULL * XP_DUMP_MAXPARTS, eb))
@@ -2939,7 +2948,7 @@ xpuhip_session_close(xpuhip_session *s)
     if (s->d_params) g_pool.free(s->d_params);
     if (s->d_xids) g_pool.free(s->d_xids);
     if (s->d_sort) g_pool.free(s->d_sort);
-    if (s->d_sort_stage) (void)hipFree(s->d_sort_stage);
+    if (s->d_sort_stage) g_pool.free(s->d_sort_stage);
     for (int d = 0; d <= XP_MAX_DEPTH; d++)
         if (s->d_inner_own[d]) g_pool.free(s->d_inner_own[d]);
     delete s;
