@@ -2860,7 +2860,12 @@ gb_num_keys(cplan *P)
 
 /* whether the group tuple holds the key registers' values.  Written without
  * early exits: the answer is one flag every lane computes to the end, not a
- * value carried out of divergent branches. */
+ * value carried out of divergent branches.  Nothing is read through pos once
+ * the flag is false: pos is the place of the next key only as long as every
+ * key so far was the tuple's own.  Tuples of other groups do come here
+ * without a hash collision: the hash leaves NULL keys out, so (V, NULL, 'x')
+ * and (NULL, V, 'x') share theirs, and a text's length word read from inside
+ * V leads as far as 1 GiB past the tuple. */
 __device__ __forceinline__ bool
 gb_keys_match(cplan *P, const Lane &L, const kern_tupitem *t)
 {
@@ -2877,27 +2882,26 @@ gb_keys_match(cplan *P, const Lane &L, const kern_tupitem *t)
         const bool tnull = !((gld<uint8_t>(&t->t_bits[j >> 3]) >> (j & 7)) & 1);
         const bool lnull = RNULL(L, ka.reg);
         same = same && tnull == lnull;      /* NULLs group together (kmode_compare_nulls) */
-        if (tnull || lnull)
+        if (!same || tnull)
             continue;
         const char *p = base + pos;
         const int64_t v = L.R[ka.reg];
         switch (ka.width)
         {
-            case 1: same = same && gld<int8_t>(p) == (int8_t)v; pos += 1; break;
-            case 2: same = same && gld<int16_t>(p) == (int16_t)v; pos += 2; break;
+            case 1: same = gld<int8_t>(p) == (int8_t)v; pos += 1; break;
+            case 2: same = gld<int16_t>(p) == (int16_t)v; pos += 2; break;
             case 4:
                 if (ka.domain == XD_F32)
-                    same = same && fcmp(XC_EQ, (double)__int_as_float(gld<int32_t>(p)),
-                                        (double)as_f32(v));
+                    same = fcmp(XC_EQ, (double)__int_as_float(gld<int32_t>(p)), (double)as_f32(v));
                 else
-                    same = same && gld<int32_t>(p) == (int32_t)v;
+                    same = gld<int32_t>(p) == (int32_t)v;
                 pos += 4;
                 break;
             case 8:
                 if (ka.domain == XD_F64)
-                    same = same && fcmp(XC_EQ, __longlong_as_double(gld<int64_t>(p)), as_f64(v));
+                    same = fcmp(XC_EQ, __longlong_as_double(gld<int64_t>(p)), as_f64(v));
                 else
-                    same = same && gld<int64_t>(p) == v;
+                    same = gld<int64_t>(p) == v;
                 pos += 8;
                 break;
             default:
@@ -2906,8 +2910,8 @@ gb_keys_match(cplan *P, const Lane &L, const kern_tupitem *t)
                 {
                     /* numeric keys group by value (xpu_numeric_datum_comp) */
                     xnum x, y;
-                    same = same && !num_parse((const uint8_t *)p, &x) &&
-                           !num_read(L, ka.reg, &y) && num_compare(x, y) == 0;
+                    same = !num_parse((const uint8_t *)p, &x) && !num_read(L, ka.reg, &y) &&
+                           num_compare(x, y) == 0;
                     pos += varsize_any((const uint8_t *)p);
                     break;
                 }
@@ -2923,7 +2927,7 @@ gb_keys_match(cplan *P, const Lane &L, const kern_tupitem *t)
                         hdr |= (uint32_t)gld<uint8_t>(p + i) << (8 * i);
                 }
                 const uint32_t tlen = ((hdr >> 2) & 0x3fffffff) - 4;
-                same = same && tlen == len;
+                same = tlen == len;
                 const uint32_t n = same ? len : 0;
                 uint32_t diff = 0;
                 if (ka.attalign >= 4)

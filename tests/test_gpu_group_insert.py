@@ -182,3 +182,39 @@ def test_batch_of_text_keys(gpu, jit):
         assert_groups_equal(s.final(), run_oracle_groupby(blob, [part]), acts)
         s.close()
     dev.free()
+
+
+@pytest.mark.parametrize("third", ["text", "numeric"])
+def test_null_keys_before_variable_length_keys(gpu, jit, third):
+    """Groups that differ in which of their int8 keys is NULL hash alike (NULLs
+    stay out of the hash) and share a chain: a walk compares each with the
+    others' tuples, whose texts and numerics lie behind different bytes.  The
+    int8 values are timestamps in microseconds, whose bytes would be lengths of
+    hundreds of MB.  Each group is there once, over heap pages and (no
+    numeric) an Arrow chunk."""
+    r = np.random.default_rng(6)
+    n = 20_000
+    base = 1_733_400_000_000_000 + r.integers(0, 12, size=n)
+    which = r.integers(0, 4, size=n)
+    pick = r.integers(0, 9, size=n)
+    short = third == "numeric"
+    var = [kds.numeric_image(str(i % 3) + ".25", short_varlena=True) if short else b"x" * (i % 3)
+           for i in pick]
+    cols = [kds.Column("a", "int8", base, (which & 1) != 0),
+            kds.Column("d", "int8", base, (which & 2) != 0),
+            kds.Column("t", third, var, r.random(n) < 0.1),
+            kds.Column("u", "text", [b"y" * (i // 3) for i in pick], r.random(n) < 0.1),
+            kds.Column("e", "int8", base + which, r.random(n) < 0.5)] + _args(n, r)
+    names = ["a", "d", "t", "u", "e"]
+    plan = cg.Plan([(c.name, c.typname) for c in cols])
+    tlist = [(abi.KAGG_ACTION__NROWS_ANY, None, ("n", "int8")),
+             (abi.KAGG_ACTION__PSUM_INT64, plan.scan_var("v"), ("sv", "bytea"))]
+    tlist += [(abi.KAGG_ACTION__VREF, plan.scan_var(k), (k, third if k == "t" else c.typname))
+              for k, c in zip(names, cols)]
+    plan.set_groupby(tlist)
+    blob = plan.build(final_nrows=5000)
+    chunks = [kds.build_block_kds(cols)] + ([] if short else [kds.build_arrow_kds(cols)])
+    for src in chunks:
+        fin = run_gpu_groupby(blob, [src, src], tuning=dict(jit=jit))
+        got = assert_groups_equal(fin, run_oracle_groupby(blob, [src, src]), [t[0] for t in tlist])
+        assert len(got) > 1000
