@@ -4408,8 +4408,9 @@ lds_flush_units(cplan *P, Lane &L, LdsTable &T, const kern_data_store *kds_src,
             base += 64;
             if (end >= 64 || last)
             {
-                entry = lane < nq ? queue : moved;
+                /* (what else a lane was sent may lie past the table) */
                 nb = end < 64 ? end : 64;
+                entry = lane >= nb ? 0 : lane < nq ? queue : moved;
                 nq = end > 64 ? end - 64 : 0;
                 queue = moved;
                 if (nb == 0)
