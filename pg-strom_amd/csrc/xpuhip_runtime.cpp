@@ -32,6 +32,7 @@
 
 #include "xpuhip.h"
 #include "xpu_compile.h"
+#include "xpu_devpool.h"
 #include "xpu_jit.h"
 #include "xpu_kernels.h"
 
@@ -134,103 +135,32 @@ ensure_device(kern_errorbuf *eb)
     return 0;
 }
 
-/* Device buffers of closed sessions, kept for the next ones: a backend opens
- * a session per query, and giving its buffers (a 1 GiB kds_final and its
- * overflow table among them) back to the driver makes the next hipMalloc of
- * that size wait until the driver has cleared the freed memory (a 2M-row
- * star query opened and closed in a row: 42 ms a query, 1.9 ms with the
- * buffers kept).  Buffers are reused
- * by device and rounded size; at most DEVPOOL_KEEP_BYTES stay idle, all go back when an
- * allocation fails or at xpuhip_shutdown.  A buffer is given back only after
- * the work that used it has completed (every entry point waits for its own). */
-#define DEVPOOL_KEEP_BYTES      (8ULL << 30)
-#define DEVPOOL_KEEP_COUNT      1024
-
-struct DevPool
+/* device memory of the pool of closed sessions' buffers */
+struct HipMem
 {
-    std::mutex  lock;
-    typedef std::pair<int, size_t> Key;             /* device, rounded size */
-    std::map<void *, Key> live;
-    std::multimap<Key, void *> idle;
-    size_t      idle_bytes = 0;
+    typedef hipError_t Error;
+    static constexpr hipError_t OUT_OF_MEMORY = hipErrorOutOfMemory;
 
-    /* at most an eighth more than asked for */
-    static size_t
-    round_up(size_t n)
+    static int
+    device()
     {
-        size_t step = 256;
-        while (step * 16 <= n)
-            step <<= 1;
-        return (n + step - 1) & ~(step - 1);
+        return g_dev.id;
     }
-    hipError_t
+    static hipError_t
     alloc(void **p, size_t n)
     {
-        const size_t sz = round_up(n);
-        const Key key(g_dev.id, sz);
-        {
-            std::lock_guard<std::mutex> g(lock);
-            auto it = idle.find(key);
-            if (it != idle.end())
-            {
-                *p = it->second;
-                idle.erase(it);
-                idle_bytes -= sz;
-                live[*p] = key;
-                return hipSuccess;
-            }
-        }
-        hipError_t rc = hipMalloc(p, sz);
-        if (rc == hipErrorOutOfMemory)
-        {
+        const hipError_t rc = hipMalloc(p, n);
+        if (rc != hipSuccess)
             (void)hipGetLastError();
-            trim();
-            rc = hipMalloc(p, sz);
-        }
-        if (rc == hipSuccess)
-        {
-            std::lock_guard<std::mutex> g(lock);
-            live[*p] = key;
-        }
         return rc;
     }
-    void
-    free(void *p)
+    static void
+    release(void *p)
     {
-        if (!p)
-            return;
-        {
-            std::lock_guard<std::mutex> g(lock);
-            auto it = live.find(p);
-            if (it != live.end())
-            {
-                const Key key = it->second;
-                const size_t sz = key.second;
-                live.erase(it);
-                if (idle_bytes + sz <= DEVPOOL_KEEP_BYTES && idle.size() < DEVPOOL_KEEP_COUNT)
-                {
-                    idle.emplace(key, p);
-                    idle_bytes += sz;
-                    return;
-                }
-            }
-        }
         (void)hipFree(p);
     }
-    void
-    trim()
-    {
-        std::multimap<Key, void *> gone;
-        {
-            std::lock_guard<std::mutex> g(lock);
-            gone.swap(idle);
-            idle_bytes = 0;
-        }
-        for (auto &e : gone)
-            (void)hipFree(e.second);
-    }
 };
-DevPool     g_pool;
+DevPool<HipMem> g_pool;
 
 /* per-call device scratch: control block, look-back words, staging */
 struct Scratch
@@ -277,7 +207,7 @@ scratch_create(Scratch *s, kern_errorbuf *eb)
            hip_ok(hipEventCreate(&s->ev0), eb, "hipEventCreate") &&
            hip_ok(hipEventCreate(&s->ev1), eb, "hipEventCreate") &&
            hip_ok(hipEventCreate(&s->evm), eb, "hipEventCreate") &&
-           hip_ok(hipMalloc((void **)&s->d_ctl, sizeof(xpu_task_ctl)), eb, "hipMalloc") &&
+           hip_ok(g_pool.alloc_direct((void **)&s->d_ctl, sizeof(xpu_task_ctl)), eb, "hipMalloc") &&
            hip_ok(hipHostMalloc((void **)&s->h_ctl, sizeof(xpu_task_ctl), hipHostMallocDefault),
                   eb, "hipHostMalloc") &&
            hip_ok(hipHostMalloc((void **)&s->h_hstat, sizeof(xheap_status), hipHostMallocDefault),
@@ -2992,7 +2922,8 @@ xpuhip_device_alloc(size_t length, void **p, kern_errorbuf *eb)
 {
     if (ensure_device(eb) != 0)
         return ERRCODE_DEVICE_ERROR;
-    return hip_ok(hipMalloc(p, length), eb, "hipMalloc") ? 0 : ERRCODE_DEVICE_ERROR;
+    /* (freed by the caller, so not from the pool) */
+    return hip_ok(g_pool.alloc_direct(p, length), eb, "hipMalloc") ? 0 : ERRCODE_DEVICE_ERROR;
 }
 
 extern "C" int
