@@ -421,9 +421,14 @@ scratch_get(xpuhip_session *s, kern_errorbuf *eb)
     return x;
 }
 
+/* a call's scratch back to its session.  A call that failed (rc) may have left
+ * work on the stream, and what the next call frees of the scratch can be
+ * another session's at once: that work ends first. */
 void
-scratch_put(xpuhip_session *s, Scratch *x)
+scratch_put(xpuhip_session *s, Scratch *x, int rc)
 {
+    if (rc != 0)
+        (void)hipStreamSynchronize(x->stream);
     std::lock_guard<std::mutex> g(s->lock);
     s->pool.push_back(x);
 }
@@ -973,7 +978,12 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
         }
     }
     if (s->d_kmrels)
+    {
+        /* attached before; an attach that failed may have left work behind */
+        if (!hip_ok(hipStreamSynchronize(nullptr), eb, "hipStreamSynchronize"))
+            return ERRCODE_DEVICE_ERROR;
         g_pool.free(s->d_kmrels);
+    }
     s->d_kmrels = nullptr;
     if (!hip_ok(g_pool.alloc((void **)&s->d_kmrels, length), eb, "hipMalloc(kmrels)") ||
         !hip_ok(hipMemcpy(s->d_kmrels, kmrels, length, hipMemcpyHostToDevice), eb, "hipMemcpy(kmrels)"))
@@ -2180,7 +2190,7 @@ xpuhip_task_exec_device_tuples(xpuhip_session *s, const kern_data_store *d_kds_s
     if (!x)
         return ERRCODE_DEVICE_ERROR;
     rc = task_exec_tuples(s, x, d_kds_src, kds_head, d_kds_dst, dst_length, resume_pos, res, eb);
-    scratch_put(s, x);
+    scratch_put(s, x, rc);
     return rc;
 }
 
@@ -2204,7 +2214,7 @@ xpuhip_task_exec_device(xpuhip_session *s, const kern_data_store *d_kds_src, uin
         rc = task_exec_pinned(s, x, d_kds_src, src_nitems, res, eb);
     else
         rc = task_exec_common(s, x, d_kds_src, src_nitems, d_kds_dst, dst_length, resume_pos, res, eb);
-    scratch_put(s, x);
+    scratch_put(s, x, rc);
     return rc;
 }
 
@@ -2462,13 +2472,13 @@ xpuhip_task_exec(xpuhip_session *s, const kern_data_store *kds_src, size_t src_l
     if (!grow(&x->d_src, &x->src_cap, kds_src->length, eb) ||
         (!preagg && !grow(&x->d_dst, &x->dst_cap, dst_length, eb)))
     {
-        scratch_put(s, x);
+        scratch_put(s, x, ERRCODE_DEVICE_ERROR);
         return ERRCODE_DEVICE_ERROR;
     }
     if (!hip_ok(hipMemcpyAsync(x->d_src, kds_src, kds_src->length, hipMemcpyHostToDevice, x->stream),
                 eb, "hipMemcpyAsync(kds_src)"))
     {
-        scratch_put(s, x);
+        scratch_put(s, x, ERRCODE_DEVICE_ERROR);
         return ERRCODE_DEVICE_ERROR;
     }
     if (tuples)
@@ -2499,7 +2509,7 @@ xpuhip_task_exec(xpuhip_session *s, const kern_data_store *kds_src, size_t src_l
                 rc = ERRCODE_DEVICE_ERROR;
         }
     }
-    scratch_put(s, x);
+    scratch_put(s, x, rc);
     return rc;
 }
 
@@ -2773,7 +2783,7 @@ xpuhip_task_final(xpuhip_session *s, kern_data_store *out, size_t length,
             memcpy((char *)out + head_len, x->h_final, 8 * nout);
             memcpy((char *)out + need - usage, x->h_final + 8 * nout, usage);
         }
-        scratch_put(s, x);
+        scratch_put(s, x, ok ? 0 : -1);
         if (!ok)
             return -1;
         return (int64_t)need;
@@ -2852,6 +2862,8 @@ xpuhip_session_close(xpuhip_session *s)
     for (Scratch *x : s->pool)
         scratch_retire(x);
     s->pool.clear();
+    /* an attach or a sort that failed may have left work on the null stream */
+    (void)hipStreamSynchronize(nullptr);
     if (s->d_plan) g_pool.free(s->d_plan);
     if (s->d_const_pool) g_pool.free(s->d_const_pool);
     if (s->d_kds_dst_head) g_pool.free(s->d_kds_dst_head);
@@ -3355,6 +3367,7 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     }
     if (rc)
     {
+        (void)hipStreamSynchronize(b->stream);      /* what was launched before it */
         hip_ok((hipError_t)rc, eb, "batch launch");
         return ERRCODE_DEVICE_ERROR;
     }
