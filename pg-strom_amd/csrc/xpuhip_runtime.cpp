@@ -247,7 +247,8 @@ scratch_destroy(Scratch *s)
 
 /* a scratch buffer of at least need bytes.  Its owner's work has completed,
  * so a buffer too small goes to the pool: hipFree would wait for every
- * stream of the process, and powers of two up to 512 MiB make few sizes. */
+ * stream of the process, and powers of two up to 512 MiB make few sizes (a
+ * device without room for that gives what is needed). */
 bool
 grow(char **p, size_t *cap, size_t need, kern_errorbuf *eb)
 {
@@ -260,10 +261,21 @@ grow(char **p, size_t *cap, size_t need, kern_errorbuf *eb)
     if (need <= (512ULL << 20))
         for (sz = 256; sz < need; sz <<= 1)
             ;
-    if (!hip_ok(g_pool.alloc((void **)p, sz), eb, "hipMalloc"))
+    hipError_t rc = g_pool.alloc((void **)p, sz);
+    if (rc == hipErrorOutOfMemory)
+        rc = g_pool.alloc((void **)p, sz = need);
+    if (!hip_ok(rc, eb, "hipMalloc"))
         return false;
     *cap = sz;
     return true;
+}
+
+/* a scratch buffer of want bytes, or of least where the device has no room
+ * for as many */
+bool
+grow_to(char **p, size_t *cap, size_t want, size_t least, kern_errorbuf *eb)
+{
+    return (least < want && grow(p, cap, want, nullptr)) || grow(p, cap, least, eb);
 }
 
 }   /* namespace */
@@ -1613,7 +1625,12 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
          * queries differ in size, and one that grows its scratch waits for
          * the driver */
         const bool large = nrows >= (1ULL << 20) && lds_nents >= 1024;
-        if (!grow((char **)&x->d_spill, &x->spill_cap, (large ? std::max(nrec, room) : nrec) * rec, eb))
+        /* what a group-by of these rows cannot do without, where the device
+         * has no room for more: a quarter of the rows, and eight tables a
+         * block; what lies beyond merges into kds_final directly */
+        const uint64_t least = std::min<uint64_t>(nrec, std::max<uint64_t>(nrows / 4, 1ULL << 20));
+        if (!grow_to((char **)&x->d_spill, &x->spill_cap, (large ? std::max(nrec, room) : nrec) * rec,
+                     least * rec, eb))
             return ERRCODE_DEVICE_ERROR;
         kp.spill = x->d_spill;
         kp.spill_cap = std::min<uint64_t>(x->spill_cap / rec, nrec + nrec / 8);
@@ -1630,7 +1647,9 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
         const uint64_t ndump = large ? dmax : std::min<uint64_t>((uint64_t)grid * lds_nents +
                                                                  std::min<uint64_t>(nrec, nrows), dmax);
         uint64_t per_part = ndump / nparts * 9 / 8 + 1024;
-        if (!grow((char **)&x->d_dump, &x->dump_cap, per_part * nparts * rw * 8, eb) ||
+        const uint64_t least_part = std::min<uint64_t>(per_part, (8ULL * grid * lds_nents) / nparts + 4096);
+        if (!grow_to((char **)&x->d_dump, &x->dump_cap, per_part * nparts * rw * 8,
+                     least_part * nparts * rw * 8, eb) ||
             !grow((char **)&x->d_dump_next, &x->dump_next_cap, 8ULL * XP_DUMP_MAXPARTS, eb))
             return ERRCODE_DEVICE_ERROR;
         kp.dump = x->d_dump;
