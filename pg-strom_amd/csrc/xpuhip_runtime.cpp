@@ -3160,8 +3160,12 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
             items.push_back(it);
         }
 
-    /* spill regions: an eighth of each fragment's rows (at least 64K records),
-     * scaled down to the batch's spill budget */
+    /* spill regions: an eighth of each fragment's rows (at least 64K records)
+     * and the records that the waves of its work items reserve ahead, scaled
+     * down to the batch's spill budget.  An item of less than 64K rows
+     * reserves more than an eighth of its rows: without room for that, most
+     * spilled rows of a batch of up to 50M rows merged into kds_final one by
+     * one (two fragments of 27M rows together: 2.9 ms; 0.88 ms with it) */
     const bool spill = P->spill_ok && lds_nents > 0;
     const uint64_t rec = spill_rec_bytes(P);
     std::vector<uint64_t> caps(ntasks, 0);
@@ -3170,7 +3174,9 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     {
         for (uint32_t f = 0; f < ntasks; f++)
         {
-            caps[f] = tasks[f].nitems / 8 > 65536 ? tasks[f].nitems / 8 : 65536;
+            const uint64_t nitems_f = ((uint64_t)tasks[f].nitems + item_rows - 1) / item_rows;
+            caps[f] = (tasks[f].nitems / 8 > 65536 ? tasks[f].nitems / 8 : 65536) +
+                      nitems_f * (block / 64) * XSPILL_CHUNK;
             spill_recs += caps[f];
         }
         if (spill_recs * rec > XBATCH_SPILL_BYTES)

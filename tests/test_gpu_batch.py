@@ -98,3 +98,25 @@ def test_batch_autotune_then_exec(frags):
         exp = run_oracle_groupby(blob, [src])
         assert_groups_equal(s.final(), exp, ACTIONS)
         s.close()
+
+
+def test_batch_small_items_have_spill_room(gpu, jit):
+    """Work items of 16K rows, of which each wave reserves spill records
+    ahead: every row without an LDS entry finds a record, none merges into
+    kds_final by itself."""
+    n = 1_500_000
+    cols = datagen.preagg_table(n)
+    src = kds.build_arrow_kds(cols)
+    d = xpuhip.DeviceBuffer(len(src), src)
+    blob = W.preagg_query(cols)
+    sess = [xpuhip.Session(blob) for _ in range(2)]
+    for s in sess:
+        s.set_tuning(jit=jit)
+    xpuhip.batch_exec([(s, d, n) for s in sess], graph=False)
+    st = xpuhip.last_task_stats()
+    assert st["spill_rows"] > 0 and st["lds_miss"] == 0, st
+    exp = run_oracle_groupby(blob, [src])
+    for s in sess:
+        assert_groups_equal(s.final(), exp, ACTIONS)
+        s.close()
+    d.free()
