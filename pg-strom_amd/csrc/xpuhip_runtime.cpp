@@ -3064,14 +3064,29 @@ batch_drop_graph(BatchScratch *b)
     b->sig.clear();
 }
 
-/* grows a device buffer; a reallocation invalidates the captured graph */
+/* grows a device buffer, to want bytes where the device has room for them; a
+ * reallocation invalidates the captured graph */
 bool
-batch_grow(BatchScratch *b, char **p, size_t *cap, size_t need, kern_errorbuf *eb)
+batch_grow(BatchScratch *b, char **p, size_t *cap, size_t need, kern_errorbuf *eb, size_t want = 0)
 {
     if (need <= *cap)
         return true;
     batch_drop_graph(b);
-    return grow(p, cap, need, eb);
+    return grow_to(p, cap, want > need ? want : need, need, eb);
+}
+
+/* the size of a batch's spill or dump buffer: from a million rows on 512 MiB,
+ * doubled as often as needed.  Batches of coalesced requests differ in size,
+ * and one larger than any before waited for gigabytes from the driver. */
+size_t
+batch_class(size_t need, uint64_t nrows)
+{
+    size_t sz = 512ULL << 20;
+    if (nrows < (1ULL << 20))
+        return need;
+    while (sz < need)
+        sz <<= 1;
+    return sz;
 }
 
 bool
@@ -3263,8 +3278,10 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
             !batch_grow(b, (char **)&b->d_sitems, &b->sitems_cap, sizeof(xbatch_sitem) * nsitems, eb) ||
             !batch_grow(b, (char **)&b->d_ctl, &b->ctl_cap, sizeof(xpu_task_ctl) * ntasks, eb) ||
             !batch_grow(b, (char **)&b->d_ticket, &b->ticket_cap, 64, eb) ||
-            (spill && !batch_grow(b, (char **)&b->d_spill, &b->spill_cap, spill_recs * rec, eb)) ||
-            (spill && !batch_grow(b, (char **)&b->d_dump, &b->dump_cap, dump_recs * rw * 8, eb)) ||
+            (spill && !batch_grow(b, (char **)&b->d_spill, &b->spill_cap, spill_recs * rec, eb,
+                                  batch_class(spill_recs * rec, total))) ||
+            (spill && !batch_grow(b, (char **)&b->d_dump, &b->dump_cap, dump_recs * rw * 8, eb,
+                                  batch_class(dump_recs * rw * 8, total))) ||
             (spill && !batch_grow(b, (char **)&b->d_dump_next, &b->dump_next_cap,
                                   8ULL * nparts * ntasks, eb)))
             return ERRCODE_DEVICE_ERROR;
@@ -3274,10 +3291,11 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
                 (void)hipHostFree(b->h_ctl);
             b->h_ctl = nullptr;
             b->hctl_cap = 0;
-            if (!hip_ok(hipHostMalloc((void **)&b->h_ctl, sizeof(xpu_task_ctl) * ntasks,
-                                      hipHostMallocDefault), eb, "hipHostMalloc"))
+            const size_t bytes = sizeof(xpu_task_ctl) * (((size_t)ntasks + 63) & ~(size_t)63);
+            if (!hip_ok(hipHostMalloc((void **)&b->h_ctl, bytes, hipHostMallocDefault), eb,
+                        "hipHostMalloc"))
                 return ERRCODE_DEVICE_ERROR;
-            b->hctl_cap = sizeof(xpu_task_ctl) * ntasks;
+            b->hctl_cap = bytes;
         }
         std::vector<xbatch_frag> frags(ntasks);
         uint64_t off = 0, doff = 0;
