@@ -483,6 +483,30 @@ lds_nents_within(const xplan *P, size_t budget)
     return (uint32_t)(n > (1U << 20) ? (1U << 20) : n);
 }
 
+/* LDS of the scan + group-by passes beside their table, at most (3,344 bytes:
+ * dump counters and bases) */
+#define XP_SCAN_STATIC_LDS      4096
+
+size_t
+scan_table_budget()
+{
+    return g_dev.lds_per_block > XP_SCAN_STATIC_LDS ? g_dev.lds_per_block - XP_SCAN_STATIC_LDS : 0;
+}
+
+/* the table of a scan + group-by launch tuned to nents entries: one of a
+ * block's whole LDS is cut to what the passes leave of it (a launch beyond
+ * it faults); a larger one is refused by the caller */
+uint32_t
+scan_table_nents(const xplan *P, uint32_t nents)
+{
+    if (!P->lds_fast)
+        return 0;
+    const size_t bytes = lds_bytes_for(P, nents);
+    if (bytes > scan_table_budget() && bytes <= g_dev.lds_per_block)
+        return lds_nents_within(P, scan_table_budget());
+    return nents;
+}
+
 /* default launch shape per task kind (the autotuner overrides it) */
 void
 default_tuning(const xpuhip_session *s, xpuhip_tuning *t)
@@ -498,8 +522,7 @@ default_tuning(const xpuhip_session *s, xpuhip_tuning *t)
         t->block_size = XP_AGG_BLOCK_MAX;
         t->rows_per_thread = 4;
         t->blocks_per_cu = 1;
-        size_t budget = g_dev.lds_per_block > 4096 ? g_dev.lds_per_block - 4096 : 0;
-        t->lds_nents = lds_nents_within(P, budget);
+        t->lds_nents = lds_nents_within(P, scan_table_budget());
     }
     else if (s->comp.has_groupby)
     {
@@ -1561,6 +1584,8 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
     if (sproj && grid > (ntiles + block / 64 - 1) / (block / 64))
         grid = (ntiles + block / 64 - 1) / (block / 64);
     uint32_t lds_nents = (preagg && P->lds_fast) ? t.lds_nents : 0;
+    if (scan_agg)
+        lds_nents = scan_table_nents(P, lds_nents);
     const bool spill = scan_agg && P->spill_ok && lds_nents > 0;
     if (scan_agg && lds_nents > 0)
     {
@@ -2335,7 +2360,7 @@ xpuhip_task_exec_device_noalloc(xpuhip_session *s, const kern_data_store *d_src,
         grid = grid < by_rows ? grid : by_rows;
     }
     grid = grid < ntiles ? grid : ntiles;
-    uint32_t lds_nents = (preagg && P->lds_fast) ? t.lds_nents : 0;
+    uint32_t lds_nents = preagg ? scan_table_nents(P, t.lds_nents) : 0;
     size_t lds = lds_bytes_for(P, lds_nents);
     if (lds + (scan_agg ? 0 : XP_PIPELINE_STATIC_LDS) > g_dev.lds_per_block)
     {
@@ -3137,7 +3162,7 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     uint32_t block = t.block_size ? t.block_size : 512;
     const uint32_t rpt = t.rows_per_thread >= 4 ? 4 : (t.rows_per_thread == 2 ? 2 : 1);
     const uint32_t grid = (uint32_t)g_dev.ncu * (t.blocks_per_cu ? t.blocks_per_cu : 1);
-    const uint32_t lds_nents = P->lds_fast ? t.lds_nents : 0;
+    const uint32_t lds_nents = scan_table_nents(P, t.lds_nents);
     const size_t lds = lds_bytes_for(P, lds_nents);
     if (lds > g_dev.lds_per_block)
     {
@@ -3520,8 +3545,7 @@ tuning_candidates(const xpuhip_session *s)
         t.rows_per_thread = rpt;
         t.blocks_per_cu = bpc;
         t.jit = s->tuning.jit;
-        size_t budget = g_dev.lds_per_block > 4096 ? g_dev.lds_per_block - 4096 : 0;
-        t.lds_nents = lds_nents_within(P, (size_t)(budget * lds_frac / bpc));
+        t.lds_nents = lds_nents_within(P, (size_t)(scan_table_budget() * lds_frac / bpc));
         if (P->lds_fast && t.lds_nents == 0)
             return;
         c.push_back(t);

@@ -120,3 +120,30 @@ def test_batch_small_items_have_spill_room(gpu, jit):
         assert_groups_equal(s.final(), exp, ACTIONS)
         s.close()
     d.free()
+
+
+@pytest.mark.parametrize("left", [200, 2000, 4000])
+@pytest.mark.parametrize("how", ["batch", "task", "noalloc"])
+def test_table_of_nearly_all_lds(frags, jit, how, left):
+    """A table that leaves the passes less LDS than their own is cut to what
+    fits: the launch runs and gives the oracle's groups."""
+    part = frags[2:5]
+    s = xpuhip.Session(part[0][1])
+    s.exec_device(part[0][3], part[0][0])
+    st = xpuhip.last_task_stats()       # the default table leaves 4096 bytes
+    s.close()
+    entry = st["lds_bytes"] // st["lds_nents"]
+    tuning = dict(jit=jit, lds_nents=st["lds_nents"] + (4096 - left) // entry)
+    if how == "batch":
+        finals, _ = run_batch(part, tuning, False)
+    else:
+        finals = []
+        for n, blob, _, d in part:
+            s = xpuhip.Session(blob)
+            s.set_tuning(**tuning)
+            rc = (s.exec_device if how == "task" else s.exec_device_noalloc)(d, n)[0]
+            assert rc == 0 and xpuhip.last_task_stats()["lds_bytes"] <= st["lds_bytes"]
+            finals.append(s.final())
+            s.close()
+    for (n, blob, src, _), fin in zip(part, finals):
+        assert_groups_equal(fin, run_oracle_groupby(blob, [src]), ACTIONS)
