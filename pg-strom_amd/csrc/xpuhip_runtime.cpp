@@ -2806,16 +2806,21 @@ xpuhip_task_final(xpuhip_session *s, kern_data_store *out, size_t length,
     h->nitems = (uint32_t)nout;
     h->usage = usage;
     memcpy(out, hbuf.data(), head_len);
-    if (8 * nout + usage <= XPU_FINAL_STAGE)
+    Scratch *x = 8 * nout + usage <= XPU_FINAL_STAGE ? scratch_get(s, nullptr) : nullptr;
+    if (x && !x->h_final &&
+        hipHostMalloc((void **)&x->h_final, XPU_FINAL_STAGE, hipHostMallocDefault) != hipSuccess)
+    {
+        /* without pinned memory the copies below do */
+        (void)hipGetLastError();
+        x->h_final = nullptr;
+        scratch_put(s, x, 0);
+        x = nullptr;
+    }
+    if (x)
     {
         /* small finals (10,000 groups of five aggregates: 1.4 MB) through
          * pinned memory with one wait */
-        Scratch *x = scratch_get(s, eb);
-        if (!x)
-            return -1;
         const bool ok =
-            (x->h_final || hip_ok(hipHostMalloc((void **)&x->h_final, XPU_FINAL_STAGE,
-                                                hipHostMallocDefault), eb, "hipHostMalloc")) &&
             hip_ok(hipMemcpyAsync(x->h_final, d_ridx, 8 * nout, hipMemcpyDeviceToHost, x->stream), eb,
                    "hipMemcpyAsync") &&
             (usage == 0 ||
