@@ -35,6 +35,7 @@
 #include "xpu_devpool.h"
 #include "xpu_jit.h"
 #include "xpu_kernels.h"
+#include "xpu_planreg.h"
 
 #define XERR(eb, code, msg) \
     xpu_set_error((eb), (code), "xpuhip_runtime.cpp", __LINE__, __func__, (msg))
@@ -284,21 +285,25 @@ bool xpuhip_tuned_shape(const xplan *P, xpuhip_tuning *t);
 
 struct JitFns;
 
-/* what the sessions of one plan shape share for the life of the process */
+/* what the sessions of one plan shape share */
 struct PlanShared
 {
+    /* never used twice in the process: names the shape in batch signatures */
+    const uint64_t  id = next_id.fetch_add(1, std::memory_order_relaxed);
+    static std::atomic<uint64_t> next_id;
     std::mutex      lock;
     /* the specialized kernels by (kind, param), found once: their key in the
      * code cache is the whole kernel source, which takes 0.15 ms to write out */
     std::map<int, const JitFns *> jit;
     std::atomic<uint64_t> rows{0};      /* rows its tasks have run */
 };
-static PlanShared *plan_shared(const xplan *P);
+std::atomic<uint64_t> PlanShared::next_id{1};
+static std::shared_ptr<PlanShared> plan_shared(const xplan *P);
 
 struct xpuhip_session
 {
     xpu_compiled    comp;
-    PlanShared     *shared = nullptr;
+    std::shared_ptr<PlanShared> shared;
     xplan          *d_plan = nullptr;
     char           *d_const_pool = nullptr;
     kern_data_store *d_kds_dst_head = nullptr;
@@ -1294,7 +1299,7 @@ const JitFns *
 jit_function(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
 {
     const int key = kind * 16 + param;
-    PlanShared *sh = s->shared;
+    PlanShared *sh = s->shared.get();
     {
         std::lock_guard<std::mutex> g(sh->lock);
         auto it = sh->jit.find(key);
@@ -3275,7 +3280,7 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     sig.push_back(((uint64_t)block << 32) | rpt);
     sig.push_back(((uint64_t)grid << 32) | lds_nents);
     sig.push_back(t.jit);
-    sig.push_back((uint64_t)(uintptr_t)s0->shared);
+    sig.push_back(s0->shared->id);
     sig.push_back((uint64_t)(uintptr_t)s0->d_plan);
     for (uint32_t f = 0; f < ntasks; f++)
     {
@@ -3515,15 +3520,11 @@ shape_key(const xplan *P)
 
 }   /* namespace */
 
-static PlanShared *
+static std::shared_ptr<PlanShared>
 plan_shared(const xplan *P)
 {
-    static std::map<std::string, std::unique_ptr<PlanShared>> shapes;
-    std::lock_guard<std::mutex> g(g_tune_lock);
-    auto &slot = shapes[shape_key(P)];
-    if (!slot)
-        slot.reset(new PlanShared());
-    return slot.get();
+    static PlanRegistry<PlanShared> shapes;
+    return shapes.get(shape_key(P));
 }
 
 namespace {
