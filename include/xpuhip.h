@@ -40,8 +40,10 @@ typedef struct
     uint32_t    join_passes;        /* XPUHIP_JOIN_PASSES_*: group-by joins in passes */
 } xpuhip_tuning;
 
-#define XPUHIP_JIT_AUTO     0       /* specialize chunks of >= 1,000,000 rows, and
-                                       any chunk of a plan that has run as many */
+#define XPUHIP_JIT_AUTO     0       /* specialize chunks (and batches) of >= 1,000,000
+                                       rows; smaller chunks of a plan whose tasks have
+                                       run as many once it is compiled, which a thread
+                                       of the library does meanwhile */
 #define XPUHIP_JIT_ON       1       /* always specialize */
 #define XPUHIP_JIT_OFF      2       /* always run the op interpreter */
 
@@ -66,6 +68,8 @@ typedef struct
 /* Device setup; replaces gpuservSetupGpuContext (gpu_service.c:6462-6523).
  * device < 0 selects device 0. */
 int     xpuhip_init(int device, kern_errorbuf *errbuf);
+/* Waits for the device and for a kernel being compiled, and gives idle
+ * device buffers back. */
 void    xpuhip_shutdown(void);
 
 /* OpenSession: validates and compiles the kern_session_info blob built by

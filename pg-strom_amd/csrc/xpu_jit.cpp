@@ -2,14 +2,20 @@
  * xpu_jit.cpp - per-plan specialization of the kernels with hiprtc.
  */
 #include <hip/hiprtc.h>
+#include <signal.h>
 #include <stddef.h>
 #include <stdarg.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
+#include <condition_variable>
+#include <deque>
 #include <map>
 #include <memory>
 #include <mutex>
+#include <system_error>
+#include <thread>
 
 #include "xpu_jit.h"
 
@@ -250,4 +256,137 @@ xpu_jit_code(const xplan *P, int kind, int param, std::string *log)
     if (!slot)
         slot = std::move(code);
     return slot.get();
+}
+
+/* ------------------------------------------------------------------
+ * compilation off the calling thread
+ * ------------------------------------------------------------------ */
+namespace {
+
+struct Request
+{
+    std::unique_ptr<xplan> plan;
+    int         kind;
+    int         param;
+    xpu_jit_progress state;
+};
+
+struct Compiler
+{
+    std::mutex  lock;
+    std::condition_variable cv;
+    std::deque<Request> queue;
+    std::thread thread;
+    std::mutex  stop_lock;
+    bool        stop = false;
+    bool        ended = false;          /* the process ends */
+    bool        at_exit = false;        /* the compiler is loaded, the exit handler set */
+    int         asked = 0;
+};
+
+/* never destroyed: the thread may be waiting on it while the process ends
+ * without its exit handlers */
+Compiler &g_bg = *new Compiler();
+
+void
+compile_loop()
+{
+    for (;;)
+    {
+        Request r;
+        {
+            std::unique_lock<std::mutex> lk(g_bg.lock);
+            g_bg.cv.wait(lk, [] { return g_bg.stop || !g_bg.queue.empty(); });
+            if (g_bg.stop)
+                return;
+            r = std::move(g_bg.queue.front());
+            g_bg.queue.pop_front();
+        }
+        std::string log;
+        const bool ok = xpu_jit_code(r.plan.get(), r.kind, r.param, &log) != nullptr;
+        r.state->store(ok ? XJ_STATE_READY : XJ_STATE_FAILED);
+    }
+}
+
+void
+stop_at_exit(void)
+{
+    {
+        std::lock_guard<std::mutex> g(g_bg.lock);
+        g_bg.ended = true;
+    }
+    xpu_jit_stop();
+}
+
+}   /* namespace */
+
+void
+xpu_jit_request(const xplan *P, int kind, int param, const xpu_jit_progress &state)
+{
+    std::lock_guard<std::mutex> g(g_bg.lock);
+    if (state->load() != XJ_STATE_NONE || g_bg.stop || g_bg.ended ||
+        g_bg.queue.size() >= XJ_BG_QUEUE || g_bg.asked >= XJ_BG_MAX)
+        return;
+    if (!g_bg.at_exit)
+    {
+        /* The process waits for the thread before the compiler's own exit
+         * handlers run: they are set when it is loaded, so it is loaded
+         * before ours is. */
+        hiprtcProgram prog;
+        if (hiprtcCreateProgram(&prog, "\n", "xpu_jit_load.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS)
+            return;
+        (void)hiprtcDestroyProgram(&prog);
+        if (atexit(stop_at_exit) != 0)
+            return;
+        g_bg.at_exit = true;
+    }
+    if (!g_bg.thread.joinable())
+    {
+        /* the process's signals go to its own threads */
+        sigset_t all, old;
+        sigfillset(&all);
+        for (int sig : {SIGSEGV, SIGBUS, SIGFPE, SIGILL, SIGABRT})
+            sigdelset(&all, sig);
+        pthread_sigmask(SIG_SETMASK, &all, &old);
+        try
+        {
+            g_bg.thread = std::thread(compile_loop);
+        }
+        catch (const std::system_error &)
+        {
+        }
+        pthread_sigmask(SIG_SETMASK, &old, nullptr);
+        if (!g_bg.thread.joinable())
+            return;
+    }
+    Request r;
+    r.plan.reset(new xplan(*P));
+    r.kind = kind;
+    r.param = param;
+    r.state = state;
+    state->store(XJ_STATE_QUEUED);
+    g_bg.queue.push_back(std::move(r));
+    g_bg.asked++;
+    g_bg.cv.notify_one();
+}
+
+void
+xpu_jit_stop(void)
+{
+    std::lock_guard<std::mutex> only(g_bg.stop_lock);
+    std::thread t;
+    {
+        std::lock_guard<std::mutex> g(g_bg.lock);
+        g_bg.stop = true;
+        for (Request &r : g_bg.queue)
+            r.state->store(XJ_STATE_NONE);
+        g_bg.asked -= (int)g_bg.queue.size();
+        g_bg.queue.clear();
+        t = std::move(g_bg.thread);
+        g_bg.cv.notify_one();
+    }
+    if (t.joinable())
+        t.join();
+    std::lock_guard<std::mutex> g(g_bg.lock);
+    g_bg.stop = false;
 }

@@ -13,6 +13,8 @@
  */
 #ifndef XPU_JIT_H
 #define XPU_JIT_H
+#include <atomic>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -33,5 +35,25 @@ bool xpu_jit_compile(const std::string &src, std::vector<char> *code, std::strin
 /* code object of the specialized kernel, compiled once per distinct source
  * in the process (thread-safe); nullptr with *log filled on failure */
 const std::vector<char> *xpu_jit_code(const xplan *P, int kind, int param, std::string *log);
+
+/* The same off the calling thread: a thread of the library compiles one
+ * kernel after another and says so in *state.  It makes no call to the HIP
+ * runtime.  Nothing happens if the state is not XJ_STATE_NONE, if the queue is
+ * full, or once XJ_BG_MAX kernels have been asked for in the process (each
+ * stays in the code cache); the caller may ask again. */
+enum xpu_jit_state
+{
+    XJ_STATE_NONE = 0,
+    XJ_STATE_QUEUED = 1,
+    XJ_STATE_READY = 2,     /* xpu_jit_code finds it */
+    XJ_STATE_FAILED = 3,
+};
+#define XJ_BG_QUEUE     16
+#define XJ_BG_MAX       512
+typedef std::shared_ptr<std::atomic<int>> xpu_jit_progress;
+void xpu_jit_request(const xplan *P, int kind, int param, const xpu_jit_progress &state);
+
+/* drops what is queued and waits for the kernel being compiled */
+void xpu_jit_stop(void);
 
 #endif

@@ -295,6 +295,7 @@ struct PlanShared
     /* the specialized kernels by (kind, param), found once: their key in the
      * code cache is the whole kernel source, which takes 0.15 ms to write out */
     std::map<int, const JitFns *> jit;
+    std::map<int, xpu_jit_progress> asked;      /* compiled off the calls */
     std::atomic<uint64_t> rows{0};      /* rows its tasks have run */
 };
 std::atomic<uint64_t> PlanShared::next_id{1};
@@ -703,6 +704,7 @@ xpuhip_init(int device, kern_errorbuf *eb)
 extern "C" void
 xpuhip_shutdown(void)
 {
+    xpu_jit_stop();
     std::lock_guard<std::mutex> g(g_dev_lock);
     if (g_dev.ready)
         (void)hipDeviceSynchronize();
@@ -1120,11 +1122,13 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
 #define XPU_SPILL_BYTES         (512ULL << 20)
 #define XPU_DUMP_BYTES          (512ULL << 20)
 
-/* XPUHIP_JIT_AUTO specializes chunks of at least this many rows, and every
- * chunk of a plan that has run as many in this process: a table comes as
- * 64 MB chunks of heap pages (about 900,000 rows of a 70-byte tuple), none of
- * which reaches the bound by itself (the scan passes over 990,000 rows of
- * heap pages: 0.40 ms interpreted, 0.10 ms specialized) */
+/* XPUHIP_JIT_AUTO specializes chunks of at least this many rows, and the
+ * smaller chunks of a plan that has run as many in this process: a table
+ * comes as 64 MB chunks of heap pages (about 900,000 rows of a 70-byte
+ * tuple), none of which reaches the bound by itself (the scan passes over
+ * 990,000 rows of heap pages: 0.40 ms interpreted, 0.10 ms specialized).  A
+ * small chunk does not wait for the compiler (0.5 s): it is interpreted until
+ * a thread of the library has compiled its plan */
 #define XPUHIP_JIT_AUTO_ROWS    1000000ULL
 
 /* device memory for the records of multi-pass joins, per task */
@@ -1313,6 +1317,32 @@ jit_function(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
         sh->jit[key] = f;
     }
     return f;
+}
+
+/* the kernels of XPUHIP_JIT_AUTO for chunks that are too small to wait for
+ * them: null, and asked for, until a thread of the library has compiled them */
+const JitFns *
+jit_when_ready(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
+{
+    const int key = kind * 16 + param;
+    PlanShared *sh = s->shared.get();
+    xpu_jit_progress state;
+    {
+        std::lock_guard<std::mutex> g(sh->lock);
+        auto it = sh->jit.find(key);
+        if (it != sh->jit.end())
+            return it->second;
+        xpu_jit_progress &a = sh->asked[key];
+        if (!a)
+            a = std::make_shared<std::atomic<int>>(XJ_STATE_NONE);
+        state = a;
+    }
+    const int v = state->load();
+    if (v == XJ_STATE_READY)
+        return jit_function(s, kind, param, eb);
+    if (v == XJ_STATE_NONE)
+        xpu_jit_request(&s->comp.plan, kind, param, state);
+    return nullptr;
 }
 
 }   /* namespace */
@@ -1540,11 +1570,6 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
      * exclusively); the groups that find no room in it go to the overflow
      * table */
     const bool use_ovf = preagg && P->nkeys > 0;
-    if (use_ovf && ensure_ovf(s, nrows, eb) != 0)
-        return ERRCODE_DEVICE_ERROR;
-    std::shared_lock<std::shared_mutex> final_hold;
-    if (preagg || s->d_kds_fallback)
-        final_hold = std::shared_lock<std::shared_mutex>(s->final_rw);
 
     /* the kernels specialized for the plan, or the interpreter.  Under
      * XPUHIP_JIT_AUTO a join with a group-by is specialized at any size:
@@ -1553,13 +1578,15 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
     const uint64_t seen = s->shared->rows.fetch_add(nrows, std::memory_order_relaxed) + nrows;
     const bool use_jit = t.jit == XPUHIP_JIT_ON ||
                          (t.jit != XPUHIP_JIT_OFF &&
-                          (seen >= XPUHIP_JIT_AUTO_ROWS || (preagg && P->nrels > 0)));
+                          (nrows >= XPUHIP_JIT_AUTO_ROWS || (preagg && P->nrels > 0)));
+    const bool often = t.jit == XPUHIP_JIT_AUTO && seen >= XPUHIP_JIT_AUTO_ROWS;
     hipFunction_t jfn = nullptr, jsfn = nullptr, jcount = nullptr, jwrite = nullptr, jdump = nullptr;
     const JitFns *jf = nullptr;
-    if (use_jit)
+    if (use_jit || often)
     {
-        jf = scan_agg ? jit_function(s, XJ_SCAN_AGG, (int)(rpt >= 4 ? 4 : rpt), eb)
-                      : jit_function(s, XJ_PIPELINE, preagg ? 1 : 0, eb);
+        const int kind = scan_agg ? XJ_SCAN_AGG : XJ_PIPELINE;
+        const int param = scan_agg ? (int)(rpt >= 4 ? 4 : rpt) : (preagg ? 1 : 0);
+        jf = use_jit ? jit_function(s, kind, param, eb) : jit_when_ready(s, kind, param, eb);
         if (jf)
         {
             jfn = jf->main;
@@ -1571,6 +1598,12 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
         else if (t.jit == XPUHIP_JIT_ON)
             return ERRCODE_DEVICE_ERROR;
     }
+    /* (held only now: a compile takes 0.5 s) */
+    if (use_ovf && ensure_ovf(s, nrows, eb) != 0)
+        return ERRCODE_DEVICE_ERROR;
+    std::shared_lock<std::shared_mutex> final_hold;
+    if (preagg || s->d_kds_fallback)
+        final_hold = std::shared_lock<std::shared_mutex>(s->final_rw);
     /* the interpreter's kernels take blocks of up to XP_BLOCK_MAX threads */
     const uint32_t max_block = jf ? jf->max_block : XP_BLOCK_MAX;
     if (block > max_block)
