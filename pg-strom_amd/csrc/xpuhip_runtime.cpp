@@ -1566,15 +1566,12 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
     uint32_t rpt = preagg ? (t.rows_per_thread ? t.rows_per_thread : 1) : 1;
     uint64_t nrows = nitems - row_begin;
 
-    /* group-by: a launch holds kds_final shared (growing it takes it
-     * exclusively); the groups that find no room in it go to the overflow
-     * table */
-    const bool use_ovf = preagg && P->nkeys > 0;
-
     /* the kernels specialized for the plan, or the interpreter.  Under
-     * XPUHIP_JIT_AUTO a join with a group-by is specialized at any size:
-     * its interpreter build has written some groups twice under contention
-     * (cause not found), its specialized build has not. */
+     * XPUHIP_JIT_AUTO a join with a group-by is specialized at any size: its
+     * interpreter build wrote some groups twice (half of the launches of a
+     * left-outer star join over 300,000 rows) until the chain walk kept every
+     * lane in its loop; it has not since, in 520 launches, but which of the
+     * changes made then cured it is not known */
     const uint64_t seen = s->shared->rows.fetch_add(nrows, std::memory_order_relaxed) + nrows;
     const bool use_jit = t.jit == XPUHIP_JIT_ON ||
                          (t.jit != XPUHIP_JIT_OFF &&
@@ -1598,7 +1595,10 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
         else if (t.jit == XPUHIP_JIT_ON)
             return ERRCODE_DEVICE_ERROR;
     }
-    /* (held only now: a compile takes 0.5 s) */
+    /* group-by: a launch holds kds_final shared (growing it takes it
+     * exclusively), and only now, with the compile (0.5 s) behind it; the
+     * groups that find no room in it go to the overflow table */
+    const bool use_ovf = preagg && P->nkeys > 0;
     if (use_ovf && ensure_ovf(s, nrows, eb) != 0)
         return ERRCODE_DEVICE_ERROR;
     std::shared_lock<std::shared_mutex> final_hold;

@@ -2,8 +2,6 @@
 and through the oracle on the same inputs, and compare."""
 import math
 
-import pytest
-
 import numpy as np
 
 from pgstrom import abi, kds, workloads as W, xpuhip
@@ -101,13 +99,3 @@ def project_all_query(cols, names=None, quals=None):
 def rows_of(dst):
     """(values tuple) of every row of a kds_dst, in row-index order."""
     return [r[0] for r in kds.parse_row_kds(dst)]
-
-
-def skip_interpreter_join_groupby(jit):
-    """Skips the interpreter case of a join with a group-by: that build
-    writes a group twice in some launches under contention (cause not
-    found; the plan-specialised build, which the default tuning uses for
-    these plans, has not)."""
-    if jit == xpuhip.JIT_OFF:
-        pytest.skip("known wrong result, cause not found: the interpreter build of a join "
-                    "with a group-by writes a group twice in some launches")
