@@ -1122,6 +1122,14 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
 #define XPU_SPILL_BYTES         (512ULL << 20)
 #define XPU_DUMP_BYTES          (512ULL << 20)
 
+/* The spill pass folds records in tables of the same size: one of a few
+ * entries folds next to nothing before it is dumped, and the rows then cost
+ * more as records than merged at once.  Below this many entries there are a
+ * million records (6M rows over 1M groups, all passes, with a million records
+ * and with room for all: 25.5 and 51.1 ms at 7 entries, 14.7 and 7.2 ms at
+ * 64, 13.5 and 2.7 ms at 256, 12.8 and 1.6 ms at 1,023) */
+#define XPU_SPILL_MIN_NENTS     64
+
 /* XPUHIP_JIT_AUTO specializes chunks of at least this many rows, and the
  * smaller chunks of a plan that has run as many in this process: a table
  * comes as 64 MB chunks of heap pages (about 900,000 rows of a 70-byte
@@ -1681,13 +1689,13 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
     {
         uint64_t rec = spill_rec_bytes(P);
         const uint64_t all = nrows + (uint64_t)grid * (block / 64) * XSPILL_CHUNK;
-        /* a table of a few entries folds next to nothing before it dumps */
-        const uint64_t room = lds_nents >= 1024 ? XPU_SPILL_BYTES / rec : 1ULL << 20;
+        const bool folds = lds_nents >= XPU_SPILL_MIN_NENTS;
+        const uint64_t room = folds ? XPU_SPILL_BYTES / rec : 1ULL << 20;
         const uint64_t nrec = std::min<uint64_t>(all, std::max<uint64_t>(nrows / 4, room));
         /* from a million rows on, the same buffer for any of them: a backend's
          * queries differ in size, and one that grows its scratch waits for
          * the driver */
-        const bool large = nrows >= (1ULL << 20) && lds_nents >= 1024;
+        const bool large = nrows >= (1ULL << 20) && folds;
         /* what a group-by of these rows cannot do without, where the device
          * has no room for more: a quarter of the rows, and eight tables a
          * block; what lies beyond merges into kds_final directly */
