@@ -4096,7 +4096,7 @@ gb_row_key(cplan *P, int k, const kern_data_store *kds, uint32_t row, int64_t *v
 }
 
 /* whether len bytes at p and q (any alignment) are equal; every byte is
- * compared, with the words that hold four of them read at once */
+ * compared, 16 at a time, from the aligned 8-byte words that hold them */
 __device__ __forceinline__ bool
 text_same(const uint8_t *p, const uint8_t *q, uint32_t len)
 {

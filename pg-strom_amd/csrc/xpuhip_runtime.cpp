@@ -1109,8 +1109,8 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
  * this many rows per block the merges outweigh the rows.  Where the tables
  * leave as partial-state dumps a group merges once however many blocks hold
  * it, and what a block costs is its table's set-up and its dump counters:
- * two wave tiles of the widest shape are enough (60,001 rows with NULLs, 30
- * blocks instead of 2: scan pass 1.78 -> 0.25 ms) */
+ * eight wave tiles of the widest shape (64 lanes of 4 rows) are enough (60,001
+ * rows with NULLs, 30 blocks instead of 2: scan pass 1.78 -> 0.25 ms) */
 #define XPU_MIN_ROWS_PER_BLOCK  (32ULL << 10)
 #define XPU_MIN_ROWS_PER_DUMP   (2ULL << 10)
 
@@ -1842,7 +1842,7 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
     else
         rc = xpu_launch_pipeline(&kp, P->nregs, grid, block, lds, preagg, x->stream);
     /* second pass over the spilled rows, stream-ordered after the first (it
-     * reads the spill count and kds_final's group count on the device) */
+     * reads the spill count on the device) */
     if (rc == 0 && spill)
     {
         (void)hipEventRecord(x->evm, x->stream);
