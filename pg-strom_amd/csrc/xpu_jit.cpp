@@ -110,7 +110,7 @@ xpu_jit_source(const xplan *P, int kind, int param)
          "    run(cplan *P, int begin, int end, Lane &L, const kern_data_store *__restrict__ kds,\n"
          "        uint32_t row, const xpu_kparams &kp)\n"
          "    {\n";
-    if (kind == XJ_SCAN_AGG)
+    if (kind == XJ_SCAN_AGG || kind == XJ_SCAN_BATCH)
         emit_segment(s, P, P->seg_scan.begin + P->stage_prefix, P->seg_final.end);
     else
     {
@@ -127,64 +127,51 @@ xpu_jit_source(const xplan *P, int kind, int param)
         if (P->nrels == 0)
             emit_segment(s, P, P->seg_scan.begin + P->stage_prefix, P->seg_final.end);
     }
-    s += "    }\n};\n\n";
-    append(s, "extern \"C\" __global__ void __launch_bounds__(%s)\n"
-              "xpu_jit_kernel(xpu_kparams kp)\n{\n",
-           kind == XJ_SCAN_AGG ? "XP_AGG_BLOCK_MAX" : "XP_BLOCK_MAX");
-    int nr = (P->nregs <= XP_NREGS_SMALL) ? XP_NREGS_SMALL : XP_NREGS;
-    if (kind == XJ_SCAN_AGG)
-        append(s, "    scan_agg_body<%d, %d, JitProg>((cplan *)xjit_plan, kp);\n", nr, param);
-    else
-        append(s, "    pipeline_body<%s, %d, JitProg>((cplan *)xjit_plan, kp);\n",
-               param ? "true" : "false", nr);
-    s += "}\n";
-    if (kind == XJ_PIPELINE && param && P->nrels > 0)
+    s += "    }\n};\n";
+    const int nr = (P->nregs <= XP_NREGS_SMALL) ? XP_NREGS_SMALL : XP_NREGS;
+    /* kernel name of blocks of at most bound threads running a device body */
+    auto kernel = [&](const std::string &name, const char *bound, const std::string &body) {
+        s += "\nextern \"C\" __global__ void __launch_bounds__(" + std::string(bound) + ")\n" + name +
+             "(xpu_kparams kp)\n{\n    " + body + "((cplan *)xjit_plan, kp);\n}\n";
+    };
+    const std::string n = std::to_string(nr), rpt = std::to_string(param);
+    switch (kind)
     {
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XQ_SCREEN_BLOCK)\n"
-             "xpu_jit_screen_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    join_screen_body<%d, XQ_SCREEN_RPT, JitProg>((cplan *)xjit_plan, kp);\n}\n", nr);
-        for (uint32_t d = 1; d <= P->nrels; d++)
-        {
-            append(s, "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-                      "xpu_jit_probe_kernel_%u(xpu_kparams kp)\n{\n", d);
-            append(s, "    join_probe_body<%d, JitProg, %u>((cplan *)xjit_plan, kp);\n}\n", nr, d);
-        }
-    }
-    if (kind == XJ_PIPELINE && !param && P->nrels == 0)
-    {
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-             "xpu_jit_scount_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    scan_proj_body<%d, XP_PROJ_RPT, JitProg, PM_COUNT>((cplan *)xjit_plan, kp);\n}\n", nr);
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-             "xpu_jit_swrite_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    scan_proj_body<%d, XP_PROJ_RPT, JitProg, PM_WRITE>((cplan *)xjit_plan, kp);\n}\n", nr);
-    }
-    if (kind == XJ_PIPELINE && !param)
-    {
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-             "xpu_jit_count_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    pipeline_body<false, %d, JitProg, PM_COUNT>((cplan *)xjit_plan, kp);\n}\n", nr);
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-             "xpu_jit_write_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    pipeline_body<false, %d, JitProg, PM_WRITE>((cplan *)xjit_plan, kp);\n}\n", nr);
-    }
-    if (kind == XJ_SCAN_AGG)
-    {
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-             "xpu_jit_spill_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    spill_agg_body<%d, JitProg>((cplan *)xjit_plan, kp);\n}\n", nr);
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-             "xpu_jit_dump_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    dump_merge_body<%d, JitProg>((cplan *)xjit_plan, kp);\n}\n", nr);
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_AGG_BLOCK_MAX)\n"
-             "xpu_jit_batch_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    batch_agg_body<%d, %d, JitProg>((cplan *)xjit_plan, kp);\n}\n", nr, param);
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-             "xpu_jit_batch_spill_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    batch_spill_body<%d, JitProg>((cplan *)xjit_plan, kp);\n}\n", nr);
-        s += "\nextern \"C\" __global__ void __launch_bounds__(XP_BLOCK_MAX)\n"
-             "xpu_jit_batch_merge_kernel(xpu_kparams kp)\n{\n";
-        append(s, "    batch_merge_body<%d, JitProg>((cplan *)xjit_plan, kp);\n}\n", nr);
+        case XJ_SCAN_AGG:
+            kernel("xpu_jit_kernel", "XP_AGG_BLOCK_MAX", "scan_agg_body<" + n + ", " + rpt + ", JitProg>");
+            kernel("xpu_jit_spill_kernel", "XP_BLOCK_MAX", "spill_agg_body<" + n + ", JitProg>");
+            kernel("xpu_jit_dump_kernel", "XP_BLOCK_MAX", "dump_merge_body<" + n + ", JitProg>");
+            break;
+        case XJ_SCAN_BATCH:
+            kernel("xpu_jit_batch_kernel", "XP_AGG_BLOCK_MAX",
+                   "batch_agg_body<" + n + ", " + rpt + ", JitProg>");
+            kernel("xpu_jit_batch_spill_kernel", "XP_BLOCK_MAX", "batch_spill_body<" + n + ", JitProg>");
+            kernel("xpu_jit_batch_merge_kernel", "XP_BLOCK_MAX", "batch_merge_body<" + n + ", JitProg>");
+            break;
+        case XJ_JOIN_PASSES:
+            kernel("xpu_jit_screen_kernel", "XQ_SCREEN_BLOCK",
+                   "join_screen_body<" + n + ", XQ_SCREEN_RPT, JitProg>");
+            for (uint32_t d = 1; d <= P->nrels; d++)
+                kernel("xpu_jit_probe_kernel_" + std::to_string(d), "XP_BLOCK_MAX",
+                       "join_probe_body<" + n + ", JitProg, " + std::to_string(d) + ">");
+            break;
+        default:
+            if (param)
+                kernel("xpu_jit_kernel", "XP_BLOCK_MAX", "pipeline_body<true, " + n + ", JitProg>");
+            else if (P->nrels == 0)
+            {
+                kernel("xpu_jit_scount_kernel", "XP_BLOCK_MAX",
+                       "scan_proj_body<" + n + ", XP_PROJ_RPT, JitProg, PM_COUNT>");
+                kernel("xpu_jit_swrite_kernel", "XP_BLOCK_MAX",
+                       "scan_proj_body<" + n + ", XP_PROJ_RPT, JitProg, PM_WRITE>");
+            }
+            else
+            {
+                kernel("xpu_jit_count_kernel", "XP_BLOCK_MAX",
+                       "pipeline_body<false, " + n + ", JitProg, PM_COUNT>");
+                kernel("xpu_jit_write_kernel", "XP_BLOCK_MAX",
+                       "pipeline_body<false, " + n + ", JitProg, PM_WRITE>");
+            }
     }
     return s;
 }

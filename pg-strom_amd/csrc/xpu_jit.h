@@ -20,13 +20,21 @@
 
 #include "xpu_program.h"
 
+/* Kernels compiled together are those that one task launches: with all that a
+ * plan could launch in one module, the first chunk waited twice as long
+ * (hiprtc on one core: C1's group-by 7.8 s with its batched passes, 4.5 s
+ * without; C0's scan 4.0 s with the passes for joins, 1.8 s without; C2's join
+ * 6.8 s with its one-kernel form, 2.7 s without). */
 enum xpu_jit_kind
 {
-    XJ_SCAN_AGG = 1,        /* scan_agg_body<NR, RPT> (param = RPT) */
-    XJ_PIPELINE = 2,        /* pipeline_body<PREAGG, NR> (param = PREAGG) */
+    XJ_SCAN_AGG = 1,        /* scan + group-by task: scan, spill and dump passes (param: rows a lane) */
+    XJ_PIPELINE = 2,        /* param 1: group-by over joins in one kernel; 0: the count and
+                               write passes of a projection */
+    XJ_SCAN_BATCH = 3,      /* the batched passes of a scan + group-by (param: rows a lane) */
+    XJ_JOIN_PASSES = 4,     /* group-by over joins: the screen pass and one pass per depth */
 };
 
-/* HIP source of the specialized kernel "xpu_jit_kernel" */
+/* HIP source of the specialized kernels */
 std::string xpu_jit_source(const xplan *P, int kind, int param);
 
 /* hiprtc compile for gfx950 into a code object; false with *log filled */

@@ -730,11 +730,19 @@ xpuhip_jit_prepare(const kern_session_info *session, size_t length, kern_errorbu
         return rc;
     const xplan *P = &c->plan;
     const bool scan_agg = c->has_groupby && P->nrels == 0 && P->fused;
-    const int kind = scan_agg ? XJ_SCAN_AGG : XJ_PIPELINE;
-    const int param = scan_agg ? 4 : (c->has_groupby ? 1 : 0);
-    std::string log;
-    if (!xpu_jit_code(P, kind, param, &log))
+    /* what its tasks and batches may launch */
+    std::vector<std::pair<int, int>> kinds;
+    if (scan_agg)
+        kinds = {{XJ_SCAN_AGG, 4}, {XJ_SCAN_BATCH, 4}};
+    else if (c->has_groupby && P->nrels > 0)
+        kinds = {{XJ_JOIN_PASSES, 0}, {XJ_PIPELINE, 1}};
+    else
+        kinds = {{XJ_PIPELINE, c->has_groupby ? 1 : 0}};
+    for (const auto &k : kinds)
     {
+        std::string log;
+        if (xpu_jit_code(P, k.first, k.second, &log))
+            continue;
         if (log.size() > 150)
             log.resize(150);
         XERR(eb, ERRCODE_DEVICE_ERROR, ("specialized kernel does not compile: " + log).c_str());
@@ -1249,60 +1257,52 @@ jit_load(xpuhip_session *s, int kind, int param, kern_errorbuf *eb)
         return &it->second;
     hipModule_t mod;
     JitFns f;
-    if (!hip_ok(hipModuleLoadData(&mod, code->data()), eb, "hipModuleLoadData") ||
-        !hip_ok(hipModuleGetFunction(&f.main, mod, "xpu_jit_kernel"), eb, "hipModuleGetFunction"))
+    if (!hip_ok(hipModuleLoadData(&mod, code->data()), eb, "hipModuleLoadData"))
         return nullptr;
-    if (kind == XJ_SCAN_AGG &&
-        (!hip_ok(hipModuleGetFunction(&f.spill, mod, "xpu_jit_spill_kernel"), eb,
-                 "hipModuleGetFunction") ||
-         !hip_ok(hipModuleGetFunction(&f.batch, mod, "xpu_jit_batch_kernel"), eb,
-                 "hipModuleGetFunction") ||
-         !hip_ok(hipModuleGetFunction(&f.batch_spill, mod, "xpu_jit_batch_spill_kernel"), eb,
-                 "hipModuleGetFunction") ||
-         !hip_ok(hipModuleGetFunction(&f.batch_merge, mod, "xpu_jit_batch_merge_kernel"), eb,
-                 "hipModuleGetFunction") ||
-         !hip_ok(hipModuleGetFunction(&f.dump, mod, "xpu_jit_dump_kernel"), eb,
-                 "hipModuleGetFunction")))
-        return nullptr;
-    if (kind == XJ_PIPELINE && !param &&
-        (!hip_ok(hipModuleGetFunction(&f.count, mod, "xpu_jit_count_kernel"), eb,
-                 "hipModuleGetFunction") ||
-         !hip_ok(hipModuleGetFunction(&f.write, mod, "xpu_jit_write_kernel"), eb,
-                 "hipModuleGetFunction")))
-        return nullptr;
-    if (kind == XJ_PIPELINE && !param && s->comp.plan.nrels == 0 &&
-        (!hip_ok(hipModuleGetFunction(&f.scount, mod, "xpu_jit_scount_kernel"), eb,
-                 "hipModuleGetFunction") ||
-         !hip_ok(hipModuleGetFunction(&f.swrite, mod, "xpu_jit_swrite_kernel"), eb,
-                 "hipModuleGetFunction")))
-        return nullptr;
-    if (kind == XJ_PIPELINE && param && s->comp.plan.nrels > 0)
+    const uint32_t nrels = s->comp.plan.nrels;
+    auto get = [&](hipFunction_t *fn, const char *name) {
+        return hip_ok(hipModuleGetFunction(fn, mod, name), eb, "hipModuleGetFunction");
+    };
+    bool ok = true;
+    switch (kind)
     {
-        if (!hip_ok(hipModuleGetFunction(&f.screen, mod, "xpu_jit_screen_kernel"), eb,
-                    "hipModuleGetFunction"))
-            return nullptr;
-        for (uint32_t d = 1; d <= s->comp.plan.nrels && d <= XP_MAX_DEPTH; d++)
-        {
-            char name[64];
-            snprintf(name, sizeof(name), "xpu_jit_probe_kernel_%u", d);
-            if (!hip_ok(hipModuleGetFunction(&f.probe[d], mod, name), eb, "hipModuleGetFunction"))
-                return nullptr;
-        }
+        case XJ_SCAN_AGG:
+            ok = get(&f.main, "xpu_jit_kernel") && get(&f.spill, "xpu_jit_spill_kernel") &&
+                 get(&f.dump, "xpu_jit_dump_kernel");
+            break;
+        case XJ_SCAN_BATCH:
+            ok = get(&f.batch, "xpu_jit_batch_kernel") &&
+                 get(&f.batch_spill, "xpu_jit_batch_spill_kernel") &&
+                 get(&f.batch_merge, "xpu_jit_batch_merge_kernel");
+            break;
+        case XJ_JOIN_PASSES:
+            ok = get(&f.screen, "xpu_jit_screen_kernel");
+            for (uint32_t d = 1; ok && d <= nrels && d <= XP_MAX_DEPTH; d++)
+                ok = get(&f.probe[d], ("xpu_jit_probe_kernel_" + std::to_string(d)).c_str());
+            break;
+        default:
+            ok = param ? get(&f.main, "xpu_jit_kernel")
+               : nrels == 0 ? get(&f.scount, "xpu_jit_scount_kernel") &&
+                              get(&f.swrite, "xpu_jit_swrite_kernel")
+                            : get(&f.count, "xpu_jit_count_kernel") &&
+                              get(&f.write, "xpu_jit_write_kernel");
     }
     /* a SIMD's 512 registers hold the four waves it gets of a 1024-thread
      * block only at 128 registers a wave: a kernel that was given more (the
      * compilers of different ROCm releases differ) runs narrower blocks */
-    if (kind == XJ_SCAN_AGG)
+    const hipFunction_t wide = kind == XJ_SCAN_AGG ? f.main : kind == XJ_SCAN_BATCH ? f.batch : nullptr;
+    if (ok && wide)
     {
-        for (hipFunction_t fn : {f.main, f.batch})
-        {
-            int regs = 0;
-            if (!hip_ok(hipFuncGetAttribute(&regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, fn), eb,
-                        "hipFuncGetAttribute"))
-                return nullptr;
-            if (regs > 128)
-                f.max_block = XP_BLOCK_MAX;
-        }
+        int regs = 0;
+        ok = hip_ok(hipFuncGetAttribute(&regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, wide), eb,
+                    "hipFuncGetAttribute");
+        if (regs > 128)
+            f.max_block = XP_BLOCK_MAX;
+    }
+    if (!ok)
+    {
+        (void)hipModuleUnload(mod);
+        return nullptr;
     }
     return &(g_mods[code] = f);
 }
@@ -1587,10 +1587,30 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
     const bool often = t.jit == XPUHIP_JIT_AUTO && seen >= XPUHIP_JIT_AUTO_ROWS;
     hipFunction_t jfn = nullptr, jsfn = nullptr, jcount = nullptr, jwrite = nullptr, jdump = nullptr;
     const JitFns *jf = nullptr;
+    /* a group-by over joins with the specialized kernels: a screen pass
+     * and one pass per depth, over slices of the rows sized to the record
+     * budget, or all depths in one kernel */
+    const bool may_pass = preagg && !scan_agg && P->nrels > 0 && use_jit &&
+                          t.join_passes != XPUHIP_JOIN_PASSES_OFF;
+    bool passes = false;
+    uint64_t slice = 0;
+    uint32_t rcap[XP_MAX_DEPTH + 2] = {}, rnw[XP_MAX_DEPTH + 2] = {};
+    size_t rec_bytes[2] = {};
+    if (may_pass)
+    {
+        /* (the grid of the launch below) */
+        const uint32_t b = block > XP_BLOCK_MAX ? XP_BLOCK_MAX : block;
+        const uint64_t tiles = (nrows + (uint64_t)b * rpt - 1) / ((uint64_t)b * rpt);
+        const uint32_t g = (uint32_t)std::min<uint64_t>((uint64_t)g_dev.ncu *
+                                                        (t.blocks_per_cu ? t.blocks_per_cu : 2), tiles);
+        passes = join_pass_sizes(P, s->maxdup, nrows, g, XQ_SCREEN_BLOCK / 64, &slice, rcap, rnw,
+                                 rec_bytes) &&
+                 (t.join_passes == XPUHIP_JOIN_PASSES_ON || slice >= nrows || slice >= (1ULL << 20));
+    }
     if (use_jit || often)
     {
-        const int kind = scan_agg ? XJ_SCAN_AGG : XJ_PIPELINE;
-        const int param = scan_agg ? (int)(rpt >= 4 ? 4 : rpt) : (preagg ? 1 : 0);
+        const int kind = scan_agg ? XJ_SCAN_AGG : passes ? XJ_JOIN_PASSES : XJ_PIPELINE;
+        const int param = scan_agg ? (int)(rpt >= 4 ? 4 : rpt) : preagg && !passes ? 1 : 0;
         jf = use_jit ? jit_function(s, kind, param, eb) : jit_when_ready(s, kind, param, eb);
         if (jf)
         {
@@ -1729,21 +1749,11 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
         kp.dump_nparts = nparts;
     }
 
-    /* a group-by over joins with the specialized kernels: a screen pass
-     * and one pass per depth, over slices of the rows sized to the record
-     * budget */
-    bool passes = false;
-    uint64_t slice = 0;
-    uint32_t rcap[XP_MAX_DEPTH + 2] = {}, rnw[XP_MAX_DEPTH + 2] = {};
-    if (preagg && !scan_agg && P->nrels > 0 && use_jit && t.join_passes != XPUHIP_JOIN_PASSES_OFF)
+    if (may_pass)
     {
-        size_t bytes[2];
-        passes = join_pass_sizes(P, s->maxdup, nrows, grid, XQ_SCREEN_BLOCK / 64, &slice, rcap, rnw,
-                                 bytes) &&
-                 (t.join_passes == XPUHIP_JOIN_PASSES_ON || slice >= nrows || slice >= (1ULL << 20));
         if (passes &&
-            (!grow((char **)&x->d_rec[0], &x->rec_cap[0], bytes[0], eb) ||
-             !grow((char **)&x->d_rec[1], &x->rec_cap[1], bytes[1], eb) ||
+            (!grow((char **)&x->d_rec[0], &x->rec_cap[0], rec_bytes[0], eb) ||
+             !grow((char **)&x->d_rec[1], &x->rec_cap[1], rec_bytes[1], eb) ||
              !grow((char **)&x->d_rec_cnt, &x->rec_cnt_cap, 8ULL * grid, eb)))
             return ERRCODE_DEVICE_ERROR;
         kp.screened = (kp.prefilter && kp.bloom[1] && !P->depth[1].left_outer) ? 1 : 0;
@@ -3338,7 +3348,7 @@ xpuhip_batch_exec(const xpuhip_batch_task *tasks, uint32_t ntasks, uint32_t flag
     const JitFns *jf = nullptr;
     if (t.jit != XPUHIP_JIT_OFF && (t.jit == XPUHIP_JIT_ON || total >= XPUHIP_JIT_AUTO_ROWS))
     {
-        jf = jit_function(s0, XJ_SCAN_AGG, (int)rpt, eb);
+        jf = jit_function(s0, XJ_SCAN_BATCH, (int)rpt, eb);
         if (!jf && t.jit == XPUHIP_JIT_ON)
             return ERRCODE_DEVICE_ERROR;
     }
