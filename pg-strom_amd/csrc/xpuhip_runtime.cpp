@@ -333,6 +333,8 @@ struct xpuhip_session
     char           *d_inner_own[XP_MAX_DEPTH + 1] = {};  /* inner buffers rebuilt from pinned
                                                             results (owned) */
     bool            inner_ready = false;
+    bool            null_work = false;      /* an attach or a sort runs on the null stream, or
+                                               failed there */
     char           *d_sort = nullptr;       /* GPU-Sort work space of task_final */
     size_t          sort_cap = 0;
     char           *d_sort_stage = nullptr; /* GPU-Sort LIMIT: the kept tuples, packed */
@@ -1027,13 +1029,11 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
             return ERRCODE_DEVICE_ERROR;
         }
     }
+    if (s->null_work && !hip_ok(hipStreamSynchronize(nullptr), eb, "hipStreamSynchronize"))
+        return ERRCODE_DEVICE_ERROR;
+    s->null_work = true;
     if (s->d_kmrels)
-    {
-        /* attached before; an attach that failed may have left work behind */
-        if (!hip_ok(hipStreamSynchronize(nullptr), eb, "hipStreamSynchronize"))
-            return ERRCODE_DEVICE_ERROR;
         g_pool.free(s->d_kmrels);
-    }
     s->d_kmrels = nullptr;
     if (!hip_ok(g_pool.alloc((void **)&s->d_kmrels, length), eb, "hipMalloc(kmrels)") ||
         !hip_ok(hipMemcpy(s->d_kmrels, kmrels, length, hipMemcpyHostToDevice), eb, "hipMemcpy(kmrels)"))
@@ -1109,6 +1109,7 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
     }
     if (!hip_ok(hipMemcpy(s->d_plan, P, sizeof(xplan), hipMemcpyHostToDevice), eb, "hipMemcpy(plan)"))
         return ERRCODE_DEVICE_ERROR;
+    s->null_work = false;       /* (the copy of the plan came last) */
     s->inner_ready = true;
     return 0;
 }
@@ -2636,6 +2637,8 @@ sort_final(xpuhip_session *s, uint32_t n, uint32_t nout, const uint64_t *d_ridx,
                         (wr ? 16ULL * n + 4 * ntiles + 4 + 8ULL * n + 7 * 256 : 0);
     if (need > s->sort_cap)
     {
+        if (s->null_work && !hip_ok(hipStreamSynchronize(nullptr), eb, "hipStreamSynchronize"))
+            return -1;
         if (s->d_sort)
             g_pool.free(s->d_sort);
         s->d_sort = nullptr;
@@ -2644,6 +2647,7 @@ sort_final(xpuhip_session *s, uint32_t n, uint32_t nout, const uint64_t *d_ridx,
             return -1;
         s->sort_cap = need;
     }
+    s->null_work = true;
     char *p = s->d_sort;
     auto take = [&](size_t bytes) { char *r = p; p += (bytes + 255) & ~(size_t)255; return r; };
     uint64_t *W[2] = {(uint64_t *)take(words_bytes), (uint64_t *)take(words_bytes)};
@@ -2770,6 +2774,7 @@ sort_final(xpuhip_session *s, uint32_t n, uint32_t nout, const uint64_t *d_ridx,
         (void)hipEventDestroy(e1);
         return -1;
     }
+    s->null_work = false;
     float ms = 0;
     (void)hipEventElapsedTime(&ms, e0, e1);
     (void)hipEventDestroy(e0);
@@ -2967,8 +2972,8 @@ xpuhip_session_close(xpuhip_session *s)
     for (Scratch *x : s->pool)
         scratch_retire(x);
     s->pool.clear();
-    /* an attach or a sort that failed may have left work on the null stream */
-    (void)hipStreamSynchronize(nullptr);
+    if (s->null_work)
+        (void)hipStreamSynchronize(nullptr);
     if (s->d_plan) g_pool.free(s->d_plan);
     if (s->d_const_pool) g_pool.free(s->d_const_pool);
     if (s->d_kds_dst_head) g_pool.free(s->d_kds_dst_head);
