@@ -1144,8 +1144,10 @@ xpuhip_session_attach_inner(xpuhip_session *s, const kern_multirels *kmrels, siz
  * comes as 64 MB chunks of heap pages (about 900,000 rows of a 70-byte
  * tuple), none of which reaches the bound by itself (the scan passes over
  * 990,000 rows of heap pages: 0.40 ms interpreted, 0.10 ms specialized).  A
- * small chunk does not wait for the compiler (0.5 s): it is interpreted until
- * a thread of the library has compiled its plan */
+ * small chunk does not wait for the compiler (0.8 s for C0's scan, 1.9 s for
+ * C1's group-by): it is interpreted until a thread of the library has compiled
+ * its plan (4,001 rows of C0 72 us a call until then and 58 after, 60,001 rows
+ * of C1 with NULLs 425 and 362) */
 #define XPUHIP_JIT_AUTO_ROWS    1000000ULL
 
 /* device memory for the records of multi-pass joins, per task */
@@ -1625,7 +1627,7 @@ task_exec_common(xpuhip_session *s, Scratch *x, const kern_data_store *d_src, ui
             return ERRCODE_DEVICE_ERROR;
     }
     /* group-by: a launch holds kds_final shared (growing it takes it
-     * exclusively), and only now, with the compile (0.5 s) behind it; the
+     * exclusively), and only now, with the compile (seconds) behind it; the
      * groups that find no room in it go to the overflow table */
     const bool use_ovf = preagg && P->nkeys > 0;
     if (use_ovf && ensure_ovf(s, nrows, eb) != 0)
