@@ -286,7 +286,9 @@ typedef struct xpuhip_server xpuhip_server;
 
 typedef struct
 {
-    uint64_t    hbm_budget;         /* bytes of requests admitted at once */
+    uint64_t    hbm_budget;         /* bytes of requests admitted at once (their own
+                                       hbm_bytes: task scratch and idle buffers of
+                                       closed sessions come on top) */
     uint32_t    slots;              /* jobs in flight (worker threads) */
     uint32_t    max_batch;          /* fragments coalesced into one launch */
 } xpuhip_server_config;
